@@ -27,6 +27,7 @@ SOURCES = [
     "csrc/fmx_api.cpp",
     "csrc/fmx_synth.hip",
     "csrc/fmx_model.hip",
+    "csrc/fmx_attn.hip",
     "csrc/fmx_model.cpp",
     "csrc/fmx_loader.cpp",
     "csrc/fmx_sched.cpp",

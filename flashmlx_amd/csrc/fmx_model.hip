@@ -231,18 +231,6 @@ __global__ __launch_bounds__(256) void dense_dec_kernel(DenseArgs a) {
 
 // ------------------------------------------------------------------ RoPE + cache
 
-__device__ inline int token_pos(const int32_t* offs, int off, int b, int l, int64_t max_seq) {
-  int64_t p = static_cast<int64_t>(offs ? offs[b] : off) + l;
-  return static_cast<int>(p < 0 ? 0 : (p >= max_seq ? max_seq - 1 : p));
-}
-
-// cache slot of sequence b: slots[b] (clamped to the cache) or b
-__device__ inline int64_t cache_slot(const int32_t* slots, int n_slots, int b) {
-  if (!slots) return b;
-  const int s = slots[b];
-  return s < 0 ? 0 : (s >= n_slots ? n_slots - 1 : s);
-}
-
 // One workgroup per token t = b * L + l at position p = offset(b) + l:
 // q heads rotated into q_out, k heads rotated into the layer's key cache at
 // p, v heads copied into the value cache at p. Rotation of pair (i, i + hd/2)
@@ -279,156 +267,6 @@ __global__ __launch_bounds__(256) void rope_cache_kernel(RopeArgs a) {
     const u32x4_t v = reinterpret_cast<const u32x4_t*>(row + (a.nh + a.nkv + g) * a.hd)[c];
     reinterpret_cast<u32x4_t*>(a.vc + ((slot * a.nkv + g) * a.max_seq + p) * a.hd)[c] = v;
   }
-}
-
-// ------------------------------------------------------------------ attention
-
-// One workgroup of kAttnThreads per (token t = b * L + l, q head h): keys
-// 0 .. p of kv head g = h / (nh / nkv), p = offset(b) + l (causal).
-//   s_j = scale * sum_d q_d k_jd   (fp32, d in order: exact bf16 products)
-//   e_j = exp(s_j - max s)         (fp64, the deterministic exp)
-//   out_d = sum_j e_j v_jd / sum_j e_j, both sums in fp64 over four
-//           contiguous quarters of the keys (keys in order within a quarter,
-//           fma), the quarter sums added in order; rounded once to bf16
-// (mx::fast::scaled_dot_product_attention, model.cpp:879-882). Scores: a
-// thread per key; the weighted sum: wave w takes quarter w, its lanes pairs
-// of dimensions. Forwards of several tokens per sequence, after
-// rope_cache_kernel (single-token forwards: attn_split_kernel).
-constexpr int kAttnThreads = 256;
-constexpr int kAttnWaves = kAttnThreads / kWave;
-constexpr int kAttnBatch = 32;  // keys whose value words are loaded together
-
-template <int PAIRS>
-__global__ __launch_bounds__(kAttnThreads) void attn_kernel(AttnArgs a) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t s_at[];
-  __shared__ float s_q[kAttnMaxHd];
-  __shared__ float s_max[kAttnWaves];
-  __shared__ double s_num[kAttnWaves][kAttnMaxHd];
-  __shared__ double s_den[kAttnWaves];
-  double* s_e = reinterpret_cast<double*>(s_at);
-  float* s_s = reinterpret_cast<float*>(s_at + static_cast<size_t>(a.max_seq) * 8);
-  const int t = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
-  const int b = t / a.L, l = t - b * a.L;
-  const int p = token_pos(a.offs, a.off, b, l, a.max_seq);
-  const int nk = p + 1;
-  const int rep = a.nh / a.nkv, g = h / rep;
-  const int64_t cbase = (cache_slot(a.slots, a.n_slots, b) * a.nkv + g) * a.max_seq * a.hd;
-  uint16_t* kb = a.kc + cbase;
-  uint16_t* vb = a.vc + cbase;
-  const uint16_t* qrow = a.q + (static_cast<int64_t>(t) * a.nh + h) * a.hd;
-  for (int d = tid; d < a.hd; d += kAttnThreads) s_q[d] = bf16_to_f32(qrow[d]);
-  __syncthreads();
-
-  // this wave's quarter of the keys for the weighted sum below; its first
-  // kAttnBatch value words are loaded now, so that their latency overlaps
-  // the scores
-  const int quarter = (nk + kAttnWaves - 1) / kAttnWaves;
-  const int j0 = min(wave * quarter, nk), j1 = min(j0 + quarter, nk);
-  const int npair = a.hd / 2;
-  const int jg = j1;
-  // lanes past the head's pairs read pair 0 (in bounds) and discard it
-  uint32_t vv[kAttnBatch][PAIRS];
-  int prl[PAIRS];
-#pragma unroll
-  for (int i = 0; i < PAIRS; ++i) prl[i] = (lane + kWave * i) < npair ? lane + kWave * i : 0;
-  auto load_values = [&](int jb) {
-#pragma unroll
-    for (int u = 0; u < kAttnBatch; ++u) {
-      const uint32_t* vr = reinterpret_cast<const uint32_t*>(vb + static_cast<int64_t>(min(jb + u, jg - 1)) * a.hd);
-#pragma unroll
-      for (int i = 0; i < PAIRS; ++i) vv[u][i] = vr[prl[i]];
-    }
-  };
-  if (j0 < jg) load_values(j0);
-
-  // scores, a thread per key
-  float m = -__builtin_huge_valf();
-  for (int jk = tid; jk < nk; jk += kAttnThreads) {
-    // the key row's chunks are loaded 16 at a time, then used in order
-    float acc = 0.0f;
-    const u32x4_t* kr = reinterpret_cast<const u32x4_t*>(kb + static_cast<int64_t>(jk) * a.hd);
-    const int nch = a.hd / 8;
-    for (int c0 = 0; c0 < nch; c0 += 16) {
-      u32x4_t kv[16];
-#pragma unroll
-      for (int c = 0; c < 16; ++c) kv[c] = kr[min(c0 + c, nch - 1)];
-#pragma unroll
-      for (int c = 0; c < 16; ++c) {
-        if (c0 + c < nch) {
-#pragma unroll
-          for (int mm = 0; mm < 4; ++mm) {
-            acc = __builtin_fmaf(s_q[8 * (c0 + c) + 2 * mm], bf16_to_f32(kv[c][mm] & 0xffffu), acc);
-            acc = __builtin_fmaf(s_q[8 * (c0 + c) + 2 * mm + 1], bf16_to_f32(kv[c][mm] >> 16), acc);
-          }
-        }
-      }
-    }
-    const float sc = acc * a.scale;
-    s_s[jk] = sc;
-    m = fmaxf(m, sc);
-  }
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
-  if (lane == 0) s_max[wave] = m;
-  __syncthreads();
-  m = s_max[0];
-#pragma unroll
-  for (int w = 1; w < kAttnWaves; ++w) m = fmaxf(m, s_max[w]);
-  for (int jk = tid; jk < nk; jk += kAttnThreads)
-    s_e[jk] = exp_det(static_cast<double>(s_s[jk]) - static_cast<double>(m));
-  __syncthreads();
-
-  // weighted sum: wave w over keys [j0, j1), lane over dimension pairs
-  // (2 pr, 2 pr + 1), pr = lane + 64 i; the value words of kAttnBatch keys
-  // are loaded together, then used in key order
-  double num[PAIRS][2], den = 0.0;
-#pragma unroll
-  for (int i = 0; i < PAIRS; ++i) num[i][0] = num[i][1] = 0.0;
-  for (int jb = j0; jb < jg; jb += kAttnBatch) {
-    if (jb != j0) load_values(jb);
-#pragma unroll
-    for (int u = 0; u < kAttnBatch; ++u) {
-      if (jb + u < jg) {
-        const double e = s_e[jb + u];
-        den += e;
-#pragma unroll
-        for (int i = 0; i < PAIRS; ++i) {
-          num[i][0] = __builtin_fma(e, static_cast<double>(bf16_to_f32(vv[u][i] & 0xffffu)), num[i][0]);
-          num[i][1] = __builtin_fma(e, static_cast<double>(bf16_to_f32(vv[u][i] >> 16)), num[i][1]);
-        }
-      }
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < PAIRS; ++i) {
-    const int pr = lane + kWave * i;
-    if (pr < npair) {
-      s_num[wave][2 * pr] = num[i][0];
-      s_num[wave][2 * pr + 1] = num[i][1];
-    }
-  }
-  if (lane == 0) s_den[wave] = den;
-  __syncthreads();
-
-  bool ovf = false;
-  for (int d = tid; d < a.hd; d += kAttnThreads) {
-    double nsum = s_num[0][d], dsum = s_den[0];
-#pragma unroll
-    for (int w = 1; w < kAttnWaves; ++w) {
-      nsum += s_num[w][d];
-      dsum += s_den[w];
-    }
-    const uint16_t o = f64_to_bf16(nsum / dsum);
-    const int64_t oc = static_cast<int64_t>(h) * a.hd + d;
-    a.out[static_cast<int64_t>(t) * a.ldo + oc] = o;
-    if (a.outh) {
-      ovf = ovf || bf16_f16_overflow(o);
-      a.outh[static_cast<int64_t>(t) * a.ldo + ((oc & ~7) | p8_slot(oc & 7))] =
-          static_cast<uint16_t>(bf16_to_f16_bits(o));
-    }
-  }
-  if (a.outh && __ballot(ovf) && lane == 0) atomicOr(a.flag, 1u);
 }
 
 // ------------------------------------------------------------------ split attention
@@ -861,8 +699,6 @@ hipError_t launch_rope_cache(const RopeArgs& a, int T, hipStream_t stream) {
   return hipGetLastError();
 }
 
-size_t attn_lds_bytes(int64_t max_seq) { return static_cast<size_t>(max_seq) * 12; }
-
 hipError_t launch_attn(const AttnArgs& a, int T, hipStream_t stream) {
   if (T == 0) return hipSuccess;
   if (a.qkv) {
@@ -873,13 +709,7 @@ hipError_t launch_attn(const AttnArgs& a, int T, hipStream_t stream) {
                        static_cast<size_t>(kAttnSplitMax * (keys * 12 + kAttnRound * kAttnPcStride * 4)), stream, a);
     return hipGetLastError();
   }
-  const dim3 grid(T, a.nh);
-  const size_t lds = attn_lds_bytes(a.max_seq);
-  if (a.hd <= 128)
-    hipLaunchKernelGGL((attn_kernel<1>), grid, dim3(kAttnThreads), lds, stream, a);
-  else
-    hipLaunchKernelGGL((attn_kernel<2>), grid, dim3(kAttnThreads), lds, stream, a);
-  return hipGetLastError();
+  return launch_attn_prefill(a, T, stream);
 }
 
 hipError_t launch_greedy(const GreedyArgs& a, int B, hipStream_t stream) {

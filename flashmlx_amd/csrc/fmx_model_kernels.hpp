@@ -61,6 +61,18 @@ hipError_t launch_dense_dec(const DenseArgs& a, hipStream_t stream);
 // Positions: token t = b * L + l sits at offs[b] + l (device offsets) or
 // off + l, clamped to [0, max_seq); its keys and values live in cache slot
 // slots[b] (or b).
+__device__ inline int token_pos(const int32_t* offs, int off, int b, int l, int64_t max_seq) {
+  int64_t p = static_cast<int64_t>(offs ? offs[b] : off) + l;
+  return static_cast<int>(p < 0 ? 0 : (p >= max_seq ? max_seq - 1 : p));
+}
+
+// cache slot of sequence b: slots[b] (clamped to the cache) or b
+__device__ inline int64_t cache_slot(const int32_t* slots, int n_slots, int b) {
+  if (!slots) return b;
+  const int s = slots[b];
+  return s < 0 ? 0 : (s >= n_slots ? n_slots - 1 : s);
+}
+
 struct RopeArgs {
   const uint16_t* qkv;    // [T, (nh + 2 nkv) * hd]: q heads, k heads, v heads
   int L, nh, nkv, hd;
@@ -108,7 +120,8 @@ __host__ __device__ inline int attn_split_range_keys(int64_t max_seq) {
   const int64_t r = (max_seq + kAttnSplitMax - 1) / kAttnSplitMax;
   return static_cast<int>(r > kAttnSplitKeys ? r : kAttnSplitKeys);
 }
-size_t attn_lds_bytes(int64_t max_seq);
+// forwards of several tokens per sequence, after launch_rope_cache (fmx_attn.hip)
+hipError_t launch_attn_prefill(const AttnArgs& a, int T, hipStream_t stream);
 hipError_t launch_attn(const AttnArgs& a, int T, hipStream_t stream);
 
 struct GreedyArgs {
