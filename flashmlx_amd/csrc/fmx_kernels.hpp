@@ -299,6 +299,7 @@ struct PfSet {
   const uint32_t* pass_tab;  // [max_pass][2] (see SortOut)
   int max_pass;              // passes the grid covers
   int rows_static;           // rows of the static passes
+  int pass_major;            // static passes: block order (pf_items sets it)
   int pass_rows;             // static passes: rows per pass (0: kPassRows; at most kPassRows)
   int n_exp;                 // experts in w (table values clamp to n_exp - 1)
   int rows_max;              // pass rows (table rows clamp to it)
@@ -319,7 +320,7 @@ struct PfArgs {
 };
 constexpr uint32_t kF16FlagX = 1u;  // x (gate/up input)
 constexpr uint32_t kF16FlagH = 2u;  // h (down input)
-// Fills ng / max_pass of a set; items of it.
+// Fills ng / pass_major of a set; items of it.
 int pf_items(PfSet& s, bool dual);
 size_t pf_lds_bytes(bool dual);
 hipError_t launch_pf(const PfArgs& a, bool dual, hipStream_t stream);
