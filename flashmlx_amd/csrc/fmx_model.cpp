@@ -113,11 +113,13 @@ struct Arena {
 // start: both at offsets independent of the token count), then the
 // activations
 struct ModelLayout {
-  uint32_t* flags;  // [2 L + 1]: per layer the q/k/v input and the o input, then the final norm
+  uint32_t* flags;  // [2 L + 1]: per layer the q/k/v input and the o input, then the final norm;
+                    //   then [kAttnSpreadWgs / 2] arrival counts of the attention
   float* rope;      // [P][hd/2][2]
   void* moe_ws;
   size_t moe_bytes;
   uint16_t *h, *normed, *normed_h, *qkv, *qrot, *attn, *attn_h, *moe_out;
+  double* attn_part;  // single-token attention's range sums, of the (token, head) pairs it spreads
   size_t total;
 };
 
@@ -125,7 +127,7 @@ ModelLayout model_layout(const fmx_model_config& c, int64_t T, char* base) {
   const Dims d = dims(c);
   Arena ar{base};
   ModelLayout M{};
-  M.flags = static_cast<uint32_t*>(ar.take((2 * d.L + 1) * 4));
+  M.flags = static_cast<uint32_t*>(ar.take((2 * d.L + 1 + kAttnSpreadWgs / 2) * 4));
   M.rope = static_cast<float*>(ar.take(d.P * (d.hd / 2) * 2 * 4));
   M.moe_bytes = fmx_moe_workspace_size(&c.moe, T);
   M.moe_ws = ar.take(M.moe_bytes);
@@ -137,6 +139,8 @@ ModelLayout model_layout(const fmx_model_config& c, int64_t T, char* base) {
   M.attn = static_cast<uint16_t*>(ar.take(T * d.nh * d.hd * 2));
   M.attn_h = static_cast<uint16_t*>(ar.take(T * d.nh * d.hd * 2));
   M.moe_out = static_cast<uint16_t*>(ar.take(T * d.H * 2));
+  M.attn_part = static_cast<double*>(ar.take(std::min<int64_t>(T * d.nh, kAttnSpreadWgs / 2) * kAttnSplitMax *
+                                             (kAttnSplitMaxHd + 2) * 8));
   M.total = ar.used;
   return M;
 }
@@ -337,7 +341,7 @@ int fmx_model_forward_batched(const fmx_model_config* cfg, const fmx_model_weigh
   ea.T = static_cast<int>(T);
   ea.h = M.h;
   ea.flags = M.flags;
-  ea.n_flags = static_cast<int>(2 * d.L + 1);
+  ea.n_flags = static_cast<int>(2 * d.L + 1 + kAttnSpreadWgs / 2);
   FMX_HIP(launch_embed(ea, stream));
 
   for (int64_t l = 0; l < d.L; ++l) {
@@ -416,6 +420,8 @@ int fmx_model_forward_batched(const fmx_model_config* cfg, const fmx_model_weigh
     aa.ldo = d.nh * d.hd;
     aa.outh = many ? M.attn_h : nullptr;
     aa.flag = M.flags + 2 * l + 1;
+    aa.part = fused ? M.attn_part : nullptr;
+    aa.arrived = M.flags + 2 * d.L + 1;
     FMX_HIP(launch_attn(aa, static_cast<int>(T), stream));
     // o_proj with the residual: h = h + attn . Wo^T
     FMX_RC(linear(M.attn, M.attn_h, M.flags + 2 * l + 1, T, lw.o, d.H, d.nh * d.hd, nullptr, M.h, M.h,

@@ -295,7 +295,29 @@ __global__ __launch_bounds__(256) void rope_cache_kernel(RopeArgs a) {
 //   M = max m_s, f_s = exp(m_s - M), den = sum_s f_s den_s,
 //   num_d = sum_s f_s num_s,d (fma; the first term a product),
 //   out_d = bf16(num_d / den)
-// (one range: f_0 = 1, the range's own sums). q and the new key are
+// (one range: f_0 = 1, the range's own sums).
+//
+// Spread: with few (token, head) pairs and many keys (kAttnSpreadKeys, known
+// on the device only) one workgroup per pair leaves CUs idle and is bound by
+// what one CU draws (16 heads, 3500 keys: 1.8 MB each at 40 GB/s); the
+// launch then has Z workgroups per pair, which exit but for the first on a
+// short context and on a long one form the same sums in the same order:
+// workgroup z has ranges z R .. z R + R - 1 (R = kAttnSplitMax / Z), Z waves
+// each. A range's score rounds go round its waves. A class's value sums are
+// one chain in key order, so what spreads are classes and dimensions: a wave
+// per class (Z >= 4; a lane takes 2 dimensions, a load one whole row) or per
+// two classes (Z = 2; 4 dimensions); with 8 or 16 waves per range the value
+// waves are those with the last score rounds or none. A wave's first score
+// round and value batch are in flight together, the second batch before the
+// weights. The range sums go to a.part through device-scope stores and the
+// last workgroup to arrive combines them. Measured, 16 heads of 128, one
+// sequence at 3500 keys: 45 -> 14 us per layer; a 4-layer step of one
+// sequence at 600 / 3500 keys 262 -> 236 / 367 -> 247 us, of 4 at 600 / 3500
+// 328 -> 322 / 439 -> 368, of 8 at 700 / 1500 / 3500 388 -> 385 / 417 -> 417
+// / 515 -> 487. From 512 keys on because every range is then a whole round
+// (at 400 keys and 24 layers the hand-over cost more than it saved).
+//
+// q and the new key are
 // rotated from the q/k/v row as rope_cache_kernel does; the new key and
 // value (position p, the last key of the last range) are used from LDS, and
 // the first q head of each kv group writes them into the caches (no
@@ -309,12 +331,14 @@ __device__ inline int attn_splits(int nk) {
   return min(kAttnSplitMax, (nk + kAttnSplitKeys - 1) / kAttnSplitKeys);
 }
 
+template <int Z>
 __global__ __launch_bounds__(kWave * kAttnSplitMax) void attn_split_kernel(AttnArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t s_at[];
   __shared__ float s_q[kAttnSplitMaxHd];
   __shared__ uint16_t s_knew[kAttnSplitMaxHd], s_vnew[kAttnSplitMaxHd];
   __shared__ double s_part[kAttnSplitMax][kAttnSplitMaxHd + 2];  // per range: m, den, num
   __shared__ double s_f[kAttnSplitMax];
+  __shared__ float s_wm[Z > 1 ? kAttnSplitMax : 1];
   const int t = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   const int rep = a.nh / a.nkv, g = h / rep;
@@ -338,12 +362,20 @@ __global__ __launch_bounds__(kWave * kAttnSplitMax) void attn_split_kernel(AttnA
   const int64_t cbase = (slot * a.nkv + g) * a.max_seq * a.hd;
   uint16_t* kb = a.kc + cbase;
   uint16_t* vb = a.vc + cbase;
+  // spread over the Z workgroups, or all ranges on the first
+  bool spread = false;
+  if constexpr (Z > 1) {
+    spread = nk > kAttnSpreadKeys;
+    if (!spread && blockIdx.z) return;
+  }
   // this wave's range; keys before jg come from the cache (p, the last key
   // of the last range, from LDS)
-  const bool active = wave < S;
-  const int j0 = active ? static_cast<int>(static_cast<int64_t>(nk) * wave / S) : 0;
-  const int j1 = active ? static_cast<int>(static_cast<int64_t>(nk) * (wave + 1) / S) : 0;
-  const bool last = wave == S - 1;
+  constexpr int R = kAttnSplitMax / Z;
+  const int range = spread ? static_cast<int>(blockIdx.z) * R + wave / Z : wave;
+  const bool active = range < S;
+  const int j0 = active ? static_cast<int>(static_cast<int64_t>(nk) * range / S) : 0;
+  const int j1 = active ? static_cast<int>(static_cast<int64_t>(nk) * (range + 1) / S) : 0;
+  const bool last = range == S - 1;
   const int jg = last ? j1 - 1 : j1;
   const int jclamp = max(jg - 1, 0);  // loads past the range re-read its last cached key
   // 2. the first key round (32 keys: instruction c brings keys c * kpi +
@@ -355,7 +387,8 @@ __global__ __launch_bounds__(kWave * kAttnSplitMax) void attn_split_kernel(AttnA
   const int kk = lane / nch, kch = lane % nch;   // this lane's key in it, its chunk
   const int nkin = max(1, kAttnRound / kpi);     // load instructions per round
   constexpr int kMaxKin = kAttnRound * kAttnSplitMaxHd / 8 / kWave;
-  u32x4_t kv[kMaxKin], vv[kAttnValKeys];
+  u32x4_t kv[kMaxKin];
+  uint32_t vv[4 * kAttnValKeys];
   // the cache is read once per step: non-temporal loads keep it from
   // evicting the next kernels' code and data (decoder stack, batch 8: 1.855
   // -> 1.805 ms per step; batch 1 unchanged)
@@ -368,11 +401,43 @@ __global__ __launch_bounds__(kWave * kAttnSplitMax) void attn_split_kernel(AttnA
   };
   auto load_values = [&](int jb) {
 #pragma unroll
-    for (int u = 0; u < kAttnValKeys; ++u)
-      vv[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(
+    for (int u = 0; u < kAttnValKeys; ++u) {
+      const u32x4_t w = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(
           vb + static_cast<int64_t>(min(jb + kc + 4 * u, jclamp)) * a.hd + 8 * min(dc, nch - 1)));
+#pragma unroll
+      for (int q = 0; q < 4; ++q) vv[4 * u + q] = w[q];
+    }
   };
-  if (active && j0 < jg) {
+  // spread: this wave's place in its range, its value class and dimensions
+  // dv0 .. dv0 + VD - 1, its first score round
+  constexpr int VC = Z == 2 ? 2 : 1, VD = 2 * VC;  // classes per wave, dimensions per lane
+  constexpr int VB = 32 / VC;                      // keys per class in a value batch
+  constexpr int VSUB = Z == 16 ? 8 : Z == 8 ? 4 : 0;
+  const int sub = wave % Z;
+  const bool vwave = Z == 2 || (sub >= VSUB && sub < VSUB + 4);
+  const int vcls = Z == 2 ? 2 * sub + (lane >> 5) : (sub - VSUB) & 3;
+  const int dv0 = VD * (lane % (kWave / VC));
+  const int js = spread ? j0 + kAttnRound * sub : j0, jstep = spread ? kAttnRound * Z : kAttnRound;
+  uint32_t v2[VB * VC];  // the second value batch (the first one is vv)
+  static_assert(VB * VC == 4 * kAttnValKeys, "a batch takes vv's registers");
+  auto load_spread = [&](int b, uint32_t (&v)[VB * VC]) {
+#pragma unroll
+    for (int u = 0; u < VB; ++u) {
+      const uint16_t* src =
+          vb + static_cast<int64_t>(min(j0 + vcls + 4 * (b * VB + u), jclamp)) * kAttnSplitMaxHd + dv0;
+      if constexpr (VC == 1) {
+        v[u] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(src));
+      } else {
+        const u32x2_t w = __builtin_nontemporal_load(reinterpret_cast<const u32x2_t*>(src));
+        v[VC * u] = w[0];
+        v[VC * u + VC - 1] = w[1];
+      }
+    }
+  };
+  if (spread) {
+    if (js < jg) load_keys(js);
+    if (vwave) load_spread(0, vv);
+  } else if (active && j0 < jg) {
     load_keys(j0);
     load_values(j0);
   }
@@ -413,9 +478,10 @@ __global__ __launch_bounds__(kWave * kAttnSplitMax) void attn_split_kernel(AttnA
   // 4. scores (LDS per wave: the range's fp64 weights, its fp32 scores,
   // and the chunk sums of one 32-key round)
   const int kmax = attn_split_range_keys(a.max_seq);
-  double* s_e = reinterpret_cast<double*>(s_at) + static_cast<size_t>(wave) * kmax;
+  const int lrange = spread ? wave / Z : wave;  // the range's place in LDS
+  double* s_e = reinterpret_cast<double*>(s_at) + static_cast<size_t>(lrange) * kmax;
   float* s_s = reinterpret_cast<float*>(s_at + static_cast<size_t>(kAttnSplitMax) * kmax * 8) +
-               static_cast<size_t>(wave) * kmax;
+               static_cast<size_t>(lrange) * kmax;
   float* s_pc = reinterpret_cast<float*>(s_at + static_cast<size_t>(kAttnSplitMax) * kmax * 12) +
                 static_cast<size_t>(wave) * kAttnRound * kAttnPcStride;
   float m = -__builtin_huge_valf();
@@ -424,8 +490,8 @@ __global__ __launch_bounds__(kWave * kAttnSplitMax) void attn_split_kernel(AttnA
     float qc[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) qc[e] = s_q[8 * kch + e];
-    for (int jb = j0; jb < jg; jb += kAttnRound) {
-      if (jb != j0) load_keys(jb);
+    for (int jb = js; jb < jg; jb += jstep) {
+      if (jb != js) load_keys(jb);
 #pragma unroll
       for (int c = 0; c < kMaxKin; ++c) {
         const int key = c * kpi + kk;
@@ -451,7 +517,8 @@ __global__ __launch_bounds__(kWave * kAttnSplitMax) void attn_split_kernel(AttnA
       }
       __builtin_amdgcn_wave_barrier();
     }
-    if (last && lane == (p - j0) % kAttnRound) {  // the new key, from LDS (the lane that takes key p below)
+    // the new key, from LDS (the lane that takes key p below)
+    if (last && lane == (p - j0) % kAttnRound && (!spread || sub == 0)) {
       float acc = 0.0f;
       for (int c = 0; c < nch; ++c) {
         float pc = 0.0f;
@@ -464,15 +531,107 @@ __global__ __launch_bounds__(kWave * kAttnSplitMax) void attn_split_kernel(AttnA
     }
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
+    if (Z > 1 && spread && lane == 0) s_wm[wave] = m;
     // each lane reads back only the scores it wrote
-    if (lane < kAttnRound)
+    if (!spread && lane < kAttnRound)
       for (int jk = j0 + lane; jk < j1; jk += kAttnRound)
         s_e[jk - j0] = exp_det(static_cast<double>(s_s[jk - j0]) - static_cast<double>(m));
   }
-  __syncthreads();
+  if (spread) {
+    if (vwave) load_spread(1, v2);
+    lds_barrier();  // (a __syncthreads would wait for the batches in flight)
+  } else {
+    __syncthreads();
+  }
+
+  if constexpr (Z > 1) {
+    if (spread) {
+      // the range's maximum over its waves, its weights
+#pragma unroll
+      for (int w = 0; w < Z; ++w) m = fmaxf(m, s_wm[lrange * Z + w]);
+      for (int i = sub * kWave + lane; i < j1 - j0; i += Z * kWave)
+        s_e[i] = exp_det(static_cast<double>(s_s[i]) - static_cast<double>(m));
+      lds_barrier();
+      // class sums, each class's keys in order
+      double* s_cls = reinterpret_cast<double*>(s_at + static_cast<size_t>(kAttnSplitMax) * kmax * 12);
+      if (vwave) {
+        double nv[VD], dv = 0.0;
+#pragma unroll
+        for (int i = 0; i < VD; ++i) nv[i] = 0.0;
+        auto add = [&](double e, const uint32_t* w) {
+          dv += e;
+#pragma unroll
+          for (int q = 0; q < VC; ++q) {
+            nv[2 * q] = __builtin_fma(e, static_cast<double>(bf16_to_f32(w[q] & 0xffffu)), nv[2 * q]);
+            nv[2 * q + 1] = __builtin_fma(e, static_cast<double>(bf16_to_f32(w[q] >> 16)), nv[2 * q + 1]);
+          }
+        };
+        auto batch = [&](int b, const uint32_t (&v)[VB * VC]) {
+#pragma unroll
+          for (int u = 0; u < VB; ++u) {
+            const int j = j0 + vcls + 4 * (b * VB + u);
+            if (j < jg) add(s_e[j - j0], v + VC * u);
+            // one key's conversions at a time, as below
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        };
+        batch(0, vv);
+        batch(1, v2);
+        for (int b = 2; j0 + 4 * VB * b < jg; ++b) {  // (Z = 2 only: one class's 64 keys are two batches)
+          load_spread(b, vv);
+          batch(b, vv);
+        }
+        if (last && vcls == (p - j0) % 4) {  // the new key's value, last of its class
+          uint32_t w[VC];
+#pragma unroll
+          for (int q = 0; q < VC; ++q) w[q] = reinterpret_cast<const uint32_t*>(s_vnew)[dv0 / 2 + q];
+          add(s_e[p - j0], w);
+        }
+        double* o = s_cls + static_cast<size_t>(4 * lrange + vcls) * (kAttnSplitMaxHd + 2);
+        if (dv0 == 0) o[1] = dv;
+#pragma unroll
+        for (int i = 0; i < VD; ++i) o[2 + dv0 + i] = nv[i];
+      }
+      if (lane == 0 && sub == 0) s_f[lrange] = static_cast<double>(m);
+      lds_barrier();
+      // the range sums, ((X_0 + X_1) + X_2) + X_3, to the combining workgroup
+      constexpr int RW = kAttnSplitMaxHd + 2;
+      double* part = a.part + static_cast<int64_t>(t * a.nh + h) * kAttnSplitMax * RW;
+      for (int i = tid; i < R * RW; i += kWave * kAttnSplitMax) {
+        const int lr = i / RW, d = i - lr * RW;
+        const double* c = s_cls + static_cast<size_t>(4 * lr) * RW + d;
+        const double v = d == 0 ? s_f[lr] : ((c[0] + c[RW]) + c[2 * RW]) + c[3 * RW];
+        __hip_atomic_store(part + blockIdx.z * (R * RW) + i, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      __shared__ int s_last;
+      wait_vmcnt0();  // this wave's device-scope stores have completed
+      __syncthreads();
+      if (tid == 0)
+        s_last = __hip_atomic_fetch_add(a.arrived + t * a.nh + h, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+                 static_cast<uint32_t>(Z - 1);
+      // the new key and value into the caches
+      if (blockIdx.z == 0 && h % rep == 0 && tid < a.hd) {
+        kb[static_cast<int64_t>(p) * a.hd + tid] = s_knew[tid];
+        vb[static_cast<int64_t>(p) * a.hd + tid] = s_vnew[tid];
+      }
+      lds_barrier();
+      if (!s_last) return;
+      if (tid == 0)
+        __hip_atomic_store(a.arrived + t * a.nh + h, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      double* sp = &s_part[0][0];
+      constexpr int N = kAttnSplitMax * RW, NT = kWave * kAttnSplitMax, PER = (N + NT - 1) / NT;
+      double pv[PER];
+#pragma unroll
+      for (int i = 0; i < PER; ++i)
+        pv[i] = __hip_atomic_load(part + min(tid + i * NT, N - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+      for (int i = 0; i < PER; ++i)
+        if (tid + i * NT < N) sp[tid + i * NT] = pv[i];
+    }
+  }
 
   // 5. the range's sums
-  if (active) {
+  if (active && !spread) {
     double nv[8], dv = 0.0;
 #pragma unroll
     for (int i = 0; i < 8; ++i) nv[i] = 0.0;
@@ -486,8 +645,8 @@ __global__ __launch_bounds__(kWave * kAttnSplitMax) void attn_split_kernel(AttnA
           dv += e;
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
-            nv[2 * q] = __builtin_fma(e, static_cast<double>(bf16_to_f32(vv[u][q] & 0xffffu)), nv[2 * q]);
-            nv[2 * q + 1] = __builtin_fma(e, static_cast<double>(bf16_to_f32(vv[u][q] >> 16)), nv[2 * q + 1]);
+            nv[2 * q] = __builtin_fma(e, static_cast<double>(bf16_to_f32(vv[4 * u + q] & 0xffffu)), nv[2 * q]);
+            nv[2 * q + 1] = __builtin_fma(e, static_cast<double>(bf16_to_f32(vv[4 * u + q] >> 16)), nv[2 * q + 1]);
           }
         }
         // one key's fp64 conversions at a time (converting a batch ahead
@@ -548,7 +707,7 @@ __global__ __launch_bounds__(kWave * kAttnSplitMax) void attn_split_kernel(AttnA
   if (a.outh && __ballot(ovf) && lane == 0) atomicOr(a.flag, 1u);
   // the new key and value into the caches, last: nothing after them waits
   // for the stores
-  if (h % rep == 0 && tid < a.hd) {
+  if (!spread && h % rep == 0 && tid < a.hd) {
     kb[static_cast<int64_t>(p) * a.hd + tid] = s_knew[tid];
     vb[static_cast<int64_t>(p) * a.hd + tid] = s_vnew[tid];
   }
@@ -699,14 +858,31 @@ hipError_t launch_rope_cache(const RopeArgs& a, int T, hipStream_t stream) {
   return hipGetLastError();
 }
 
+// Workgroups per (token, head) of a single-token forward: as many as the
+// CUs hold at one workgroup each, when the cache is long enough for any.
+static int attn_spread_wgs(const AttnArgs& a, int T) {
+  if (!a.part || a.hd != kAttnSplitMaxHd || a.max_seq <= kAttnSpreadKeys) return 1;
+  const int64_t pairs = static_cast<int64_t>(T) * a.nh;
+  int z = 1;
+  while (z < kAttnSplitMax && pairs * 2 * z <= kAttnSpreadWgs) z *= 2;
+  return z;
+}
+
 hipError_t launch_attn(const AttnArgs& a, int T, hipStream_t stream) {
   if (T == 0) return hipSuccess;
   if (a.qkv) {
     if (a.L != 1 || a.hd > kAttnSplitMaxHd || a.hd % 8 || kWave % (a.hd / 8)) return hipErrorInvalidValue;
     // LDS: per wave, a range's fp64 weights and fp32 scores, one round's chunk sums
     const int64_t keys = attn_split_range_keys(a.max_seq);
-    hipLaunchKernelGGL(attn_split_kernel, dim3(T, a.nh), dim3(kWave * kAttnSplitMax),
-                       static_cast<size_t>(kAttnSplitMax * (keys * 12 + kAttnRound * kAttnPcStride * 4)), stream, a);
+    const size_t lds = static_cast<size_t>(kAttnSplitMax * (keys * 12 + kAttnRound * kAttnPcStride * 4));
+    const dim3 nt(kWave * kAttnSplitMax);
+    switch (attn_spread_wgs(a, T)) {
+      case 16: hipLaunchKernelGGL(attn_split_kernel<16>, dim3(T, a.nh, 16), nt, lds, stream, a); break;
+      case 8: hipLaunchKernelGGL(attn_split_kernel<8>, dim3(T, a.nh, 8), nt, lds, stream, a); break;
+      case 4: hipLaunchKernelGGL(attn_split_kernel<4>, dim3(T, a.nh, 4), nt, lds, stream, a); break;
+      case 2: hipLaunchKernelGGL(attn_split_kernel<2>, dim3(T, a.nh, 2), nt, lds, stream, a); break;
+      default: hipLaunchKernelGGL(attn_split_kernel<1>, dim3(T, a.nh), nt, lds, stream, a);
+    }
     return hipGetLastError();
   }
   return launch_attn_prefill(a, T, stream);

@@ -108,6 +108,11 @@ struct AttnArgs {
   int64_t ldo;
   uint16_t* outh;         // null, or the same in fp16 (P8 layout); values outside fp16 set *flag
   uint32_t* flag;
+  // single-token forwards, both or neither (then one workgroup per token and
+  // head): range sums handed between workgroups and arrival counts, zero
+  // before the launch and after it
+  double* part;           // [kAttnSpreadWgs / 2][kAttnSplitMax][kAttnSplitMaxHd + 2]
+  uint32_t* arrived;      // [kAttnSpreadWgs / 2]
 };
 // single-token forwards (qkv set; head size at most kAttnSplitMaxHd): a
 // query's keys in min(kAttnSplitMax, ceil(keys / kAttnSplitKeys))
@@ -115,6 +120,11 @@ struct AttnArgs {
 constexpr int kAttnSplitMax = 16;
 constexpr int kAttnSplitKeys = 32;
 constexpr int kAttnSplitMaxHd = 128;
+// contexts of more keys than this are spread over several workgroups per
+// (token, head), as many (a power of two up to kAttnSplitMax) as keep the
+// grid within kAttnSpreadWgs
+constexpr int kAttnSpreadKeys = kAttnSplitMax * kAttnSplitKeys;
+constexpr int kAttnSpreadWgs = 256;
 // the longest range of a cache of max_seq positions
 __host__ __device__ inline int attn_split_range_keys(int64_t max_seq) {
   const int64_t r = (max_seq + kAttnSplitMax - 1) / kAttnSplitMax;
