@@ -229,6 +229,68 @@ __global__ __launch_bounds__(256) void dense_dec_kernel(DenseArgs a) {
   }
 }
 
+// The same products of a matrix with many tiles (an lm_head) and K of at most
+// 4 kDnBatch units, no epilogue: workgroup b has tiles b, b + gridDim.x, ..,
+// holds its waves' activation operands in registers across them and issues a
+// tile's weights before it multiplies the tile before, so the weight stream
+// never waits for a workgroup's start, its rows or its reduction. Bound by
+// HBM: lm_head [151936, 2048] (175 MB) 44.0 -> 34.5 us for one row (5.1 TB/s,
+// a large copy's rate), 59-61 -> 38.0 us for 8 rows, which every tile's
+// workgroup read again. From two tiles per resident workgroup on: below, a
+// workgroup has one tile or the grid one round, and nothing to overlap.
+constexpr int kDnWideWgs = 3 * 256;  // resident workgroups: 3 per CU by registers
+constexpr int kDnWideTiles = 2 * kDnWideWgs;
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void dense_wide_kernel(DenseArgs a) {
+  __shared__ f32x4_t s_acc[2][3][kWave];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int i16 = lane & 15, j = lane >> 4;
+  struct Batch {
+    PkUnit<false> u[kDnBatch];
+  };
+  auto load = [&](Batch& L, int tile) {
+    const uint8_t* tb = a.w + static_cast<int64_t>(min(tile, a.nt - 1)) * a.nu * kBlockSingle;
+#pragma unroll
+    for (int d = 0; d < kDnBatch; ++d)
+      L.u[d] = pk_load<false>(tb + static_cast<int64_t>(min(wave + 4 * d, a.nu - 1)) * kBlockSingle, lane);
+  };
+  Batch L0, L1;
+  load(L0, blockIdx.x);
+  const uint16_t* xrow = a.x + static_cast<int64_t>(min(i16, a.T - 1)) * a.ldx + 8 * j;
+  bf16x8_t A[kDnBatch][4];
+#pragma unroll
+  for (int d = 0; d < kDnBatch; ++d)
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      A[d][q] = *reinterpret_cast<const bf16x8_t*>(xrow + 128 * min(wave + 4 * d, a.nu - 1) + 32 * q);
+  auto tile_step = [&](int tile, int buf, Batch& L, Batch& Ln) {
+    load(Ln, tile + static_cast<int>(gridDim.x));  // (past the last tile: its weights again, unused)
+    __builtin_amdgcn_sched_barrier(0);
+    f32x4_t acc = {0.f, 0.f, 0.f, 0.f}, unused = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int d = 0; d < kDnBatch; ++d)
+      if (wave + 4 * d < a.nu) pk_unit<false>(L.u[d], A[d], acc, unused);
+    if (wave > 0) s_acc[buf][wave - 1][lane] = acc;
+    lds_barrier();
+    if (wave == 0) {
+#pragma unroll
+      for (int w = 0; w < 3; ++w) acc += s_acc[buf][w][lane];
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (4 * j + r < a.T) a.out[static_cast<int64_t>(4 * j + r) * a.ldo + tile * 16 + i16] = f32_to_bf16(acc[r]);
+    }
+  };
+  int tile = blockIdx.x;
+  for (;;) {
+    if (tile >= a.nt) break;
+    tile_step(tile, 0, L0, L1);
+    tile += gridDim.x;
+    if (tile >= a.nt) break;
+    tile_step(tile, 1, L1, L0);
+    tile += gridDim.x;
+  }
+}
+
 // ------------------------------------------------------------------ RoPE + cache
 
 // One workgroup per token t = b * L + l at position p = offset(b) + l:
@@ -847,6 +909,11 @@ hipError_t launch_dense_dec(const DenseArgs& a, hipStream_t stream) {
   const size_t lds = nin ? static_cast<size_t>(a.T) * a.nu * 128 * 2 : 0;
   if (nin)
     hipLaunchKernelGGL(dense_dec_kernel<true>, dim3(a.nt), dim3(256), lds, stream, a);
+  else if (a.nt >= kDnWideTiles && a.nu <= 4 * kDnBatch && !a.bias && !a.res)
+    // as many workgroups as make every one's tile count the same
+    hipLaunchKernelGGL(dense_wide_kernel, dim3((a.nt + (a.nt + kDnWideWgs - 1) / kDnWideWgs - 1) /
+                                               ((a.nt + kDnWideWgs - 1) / kDnWideWgs)),
+                       dim3(256), 0, stream, a);
   else
     hipLaunchKernelGGL(dense_dec_kernel<false>, dim3(a.nt), dim3(256), lds, stream, a);
   return hipGetLastError();
