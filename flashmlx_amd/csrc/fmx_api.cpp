@@ -542,11 +542,20 @@ int fmx_quantized_matmul(const fmx_array* x, const fmx_array* w, const fmx_array
     PfSet s = mlx_set(w, scales, biases, xr, K, N, static_cast<uint16_t*>(out->data));
     s.io_f16 = f16 ? 1 : 0;
     s.rows_static = s.rows_max = s.x_rows = static_cast<int>(rows);
-    // fewer work items than CUs: passes of 32 rows instead (twice the items,
-    // each with half the rows; Qwen1.5 shared shape [5632, 2048]: 48-256 rows
-    // 8-16 % faster, 512 rows, 352 items of 64, 9 % slower so)
-    const int64_t groups = (N / 16 + 7) / 8;
-    if (rows > 32 && ((rows + kPassRows - 1) / kPassRows) * groups < 256) s.pass_rows = 32;
+    // few work items: half the columns and at most 32 rows each, up to two
+    // items per CU (us, wide -> narrow: [5632, 2048] 45 rows 20.0 -> 17.8, 150
+    // rows 20.5 -> 18.6, 200 rows, 616 items, 22.6 -> 22.9; [2048, 5632] 45
+    // rows 37.1 -> 30.3, 512 rows 45.6 -> 41.1; [2048, 2048] 17-256 rows 18.7-
+    // 20.5 -> 16.7-18.2, 800 rows, 800 items, 27.0 -> 34.7); else, with fewer
+    // items of 64 rows than CUs, passes of 32 rows alone ([5632, 2048]: 200
+    // and 256 rows; 512 rows, 352 items of 64, 9 % slower so)
+    const int64_t nt = N / 16, groups = (nt + 7) / 8;
+    if ((rows + 31) / 32 * ((nt + 3) / 4) <= 512) {
+      s.narrow = 1;
+      s.pass_rows = 32;
+    } else if (rows > 32 && ((rows + kPassRows - 1) / kPassRows) * groups < 256) {
+      s.pass_rows = 32;
+    }
     FMX_HIP(launch_mlx_pf(s, xr, stream));
     return ok();
   }

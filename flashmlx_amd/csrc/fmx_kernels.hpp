@@ -294,6 +294,7 @@ struct PfSet {
                              //   then writes fp16 SwiGLU rows, the exact path is never taken)
   int nt;                    // 16-row tiles of the weight matrix (pairs: of gate)
   int nu;                    // 128-k units of K
+  int narrow;                // MLX sets: column groups of half the width
   int ng;                    // column groups (kPfWaves * blocks per wave tiles each)
   const uint32_t* pass_n;    // device pass count (null: static passes over rows_static)
   const uint32_t* pass_tab;  // [max_pass][2] (see SortOut)

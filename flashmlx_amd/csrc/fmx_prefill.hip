@@ -77,16 +77,17 @@ constexpr int64_t kPassMajorBytes = 3 << 20;  // weights that stay beside the ro
 // Packed blocks per wave: one gate/up pair or two single blocks (2 KB of
 // weight words per unit), so a workgroup's two stages fit three workgroups
 // in a CU's LDS.
-template <bool DUAL>
-constexpr int pf_nb() { return DUAL ? 1 : 2; }
+// NARROW (MLX-layout weights only): one single block.
+template <bool DUAL, bool NARROW = false>
+constexpr int pf_nb() { return DUAL || NARROW ? 1 : 2; }
 template <bool DUAL>
 constexpr int pf_nm() { return DUAL ? 2 : 1; }
 // a wave's share of one unit: its 1 KB weight pieces, then the blocks'
 // (scale, bias) words (256 bytes, one 4-byte DMA per lane)
-template <bool DUAL>
-constexpr int pf_wave_bbytes() { return pf_nb<DUAL>() * pf_nm<DUAL>() * 1024 + 256; }
-template <bool DUAL>
-constexpr int pf_stage_bytes() { return kPfABytes + kPfWaves * pf_wave_bbytes<DUAL>(); }
+template <bool DUAL, bool NARROW = false>
+constexpr int pf_wave_bbytes() { return pf_nb<DUAL, NARROW>() * pf_nm<DUAL>() * 1024 + 256; }
+template <bool DUAL, bool NARROW = false>
+constexpr int pf_stage_bytes() { return kPfABytes + kPfWaves * pf_wave_bbytes<DUAL, NARROW>(); }
 
 // LDS DMA instructions one wave issues per unit: its row pieces (one per
 // 16-row tile the pass fills), the 1 KB weight pieces of its blocks and one
@@ -104,13 +105,13 @@ __device__ inline void dma4(const void* g, void* lds) {
 // One unit's products: the pass's rows in LDS at sa (16-byte chunks
 // XOR-swizzled by row), the wave's packed words W and (scale, bias) pairs
 // SB, accumulated into acc.
-template <bool DUAL, int MT, bool F16, bool MLX>
+template <bool DUAL, int MT, bool F16, bool MLX, bool NARROW>
 __device__ __attribute__((always_inline)) void pf_unit(const PfSet& P, const uint8_t* sa,
-                                                       const u32x4_t (&W)[pf_nb<DUAL>()][pf_nm<DUAL>()],
-                                                       const u32x2_t (&SB)[pf_nb<DUAL>()][pf_nm<DUAL>()],
-                                                       f32x4_t (&acc)[MT][pf_nb<DUAL>()][pf_nm<DUAL>()], int i16,
+                                                       const u32x4_t (&W)[pf_nb<DUAL, NARROW>()][pf_nm<DUAL>()],
+                                                       const u32x2_t (&SB)[pf_nb<DUAL, NARROW>()][pf_nm<DUAL>()],
+                                                       f32x4_t (&acc)[MT][pf_nb<DUAL, NARROW>()][pf_nm<DUAL>()], int i16,
                                                        int j) {
-  constexpr int NB = pf_nb<DUAL>(), NM = pf_nm<DUAL>();
+  constexpr int NB = pf_nb<DUAL, NARROW>(), NM = pf_nm<DUAL>();
   if constexpr (F16) {
     // every activation operand of the unit is read up front (one LDS round
     // trip per unit, not one per k-slice)
@@ -211,12 +212,12 @@ __device__ __attribute__((always_inline)) void pf_unit(const PfSet& P, const uin
 // of the Qwen1.5 block at 512 / 4096 tokens 50.9 / 260 -> 46.9 / 237 us;
 // stack prefill of 3001 tokens 1.78 -> 1.68 ms; quantized_matmul of 45 rows
 // 21.0 -> 19.2 us, gather_qmm of 301 tokens 53.4 -> 49.6).
-template <bool DUAL, int MT, bool MLX>
+template <bool DUAL, int MT, bool MLX, bool NARROW>
 __device__ __attribute__((always_inline)) void pf_epilogue(const PfSet& P,
-                                                           f32x4_t (&acc)[MT][pf_nb<DUAL>()][pf_nm<DUAL>()],
+                                                           f32x4_t (&acc)[MT][pf_nb<DUAL, NARROW>()][pf_nm<DUAL>()],
                                                            int tile0, int row0, int rows, int ks, int i16, int j,
                                                            int lane, uint32_t* flag, uint32_t flag_out) {
-  constexpr int NB = pf_nb<DUAL>(), NM = pf_nm<DUAL>();
+  constexpr int NB = pf_nb<DUAL, NARROW>(), NM = pf_nm<DUAL>();
   bool ovf = false;
   // f(acc[mt][b], rows 16 mt + 4j + r, their output rows' first elements,
   // column, its place in the P8 layout) for every tile of the matrix
@@ -336,18 +337,18 @@ __device__ __attribute__((always_inline)) void pf_epilogue(const PfSet& P,
 // weights, column group ng. MT (the 16-row tiles the rows fill) fixes how
 // many row pieces each wave moves per unit, so the pass's rows are moved
 // and multiplied once, without padding to kPassRows.
-template <bool DUAL, int MT, bool F16, bool MLX>
+template <bool DUAL, int MT, bool F16, bool MLX, bool NARROW>
 __device__ __attribute__((always_inline)) void pf_item(const PfSet& P, int ng, int row0, int rows,
                                                        int64_t e, int ks, uint8_t* s_pf,
                                                        uint32_t* flag, uint32_t flag_out) {
-  constexpr int NB = pf_nb<DUAL>(), NM = pf_nm<DUAL>();
+  constexpr int NB = pf_nb<DUAL, NARROW>(), NM = pf_nm<DUAL>();
   constexpr int BB = DUAL ? kBlockPair : kBlockSingle;
   constexpr int PA = (4 * MT + kPfWaves - 1) / kPfWaves;  // 4-row pieces per wave and unit
   constexpr int PER = PA + NB * NM + 1;                  // LDS DMA instructions per wave and unit
-  constexpr int WB = pf_wave_bbytes<DUAL>(), SBO = NB * NM * 1024;  // wave's stage share, its sb offset
-  constexpr int STAGE = pf_stage_bytes<DUAL>();
-  static_assert(NB * NM * 128 == 256, "the blocks' (scale, bias) words fill one 4-byte DMA");
-  static_assert(!MLX || !DUAL, "MLX-layout weights: single matrices only");
+  constexpr int WB = pf_wave_bbytes<DUAL, NARROW>(), SBO = NB * NM * 1024;  // wave's stage share, its sb offset
+  constexpr int STAGE = pf_stage_bytes<DUAL, NARROW>();
+  static_assert(NB * NM * 128 == 256 || (MLX && NARROW), "the blocks' (scale, bias) words fill one 4-byte DMA");
+  static_assert((!MLX || !DUAL) && (MLX || !NARROW), "MLX-layout weights: single matrices only");
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -385,13 +386,13 @@ __device__ __attribute__((always_inline)) void pf_item(const PfSet& P, int ng, i
 
   // the (scale, bias) piece: lane l fetches 4 bytes of block l / SBL's
   // 16 x 8 (single) or 2 x 16 x 8 (pair) bytes
-  constexpr int SBL = kWave / NB;  // lanes per block
+  constexpr int SBL = MLX ? 32 : kWave / NB;  // lanes per block (NARROW: the second half repeats the block)
   const uint8_t* sb_src;
   if constexpr (MLX) {
     // the scale (even lanes) or bias (odd lanes) pair of groups 2u, 2u + 1
     // of row (lane % 32) / 2 of block lane / 32, at the place of the
     // packed block's (scale, bias) word
-    const int64_t row = static_cast<int64_t>(e) * P.nt * 16 + min(tile0 + lane / SBL, P.nt - 1) * 16 +
+    const int64_t row = static_cast<int64_t>(e) * P.nt * 16 + min(tile0 + min(lane / SBL, NB - 1), P.nt - 1) * 16 +
                         (lane % SBL) / 2;
     sb_src = reinterpret_cast<const uint8_t*>((lane & 1 ? P.mb : P.ms) + row * (P.nu * 2) + 2 * kb);
   } else {
@@ -464,9 +465,9 @@ __device__ __attribute__((always_inline)) void pf_item(const PfSet& P, int ng, i
         }
         SB[b][m] = *reinterpret_cast<const u32x2_t*>(sb + SBO + b * (NM * 128) + m * 128 + 8 * i16);
       }
-    pf_unit<DUAL, MT, F16, MLX>(P, sa, W, SB, acc, i16, j);
+    pf_unit<DUAL, MT, F16, MLX, NARROW>(P, sa, W, SB, acc, i16, j);
   }
-  pf_epilogue<DUAL, MT, MLX>(P, acc, tile0, row0, rows, ks, i16, j, lane, flag, flag_out);
+  pf_epilogue<DUAL, MT, MLX, NARROW>(P, acc, tile0, row0, rows, ks, i16, j, lane, flag, flag_out);
 }
 
 // Block -> work item. The hardware dispatches block b to XCD b % 8, each
@@ -484,7 +485,7 @@ __device__ __attribute__((always_inline)) void pf_item(const PfSet& P, int ng, i
 // Otherwise it runs every pass of one group back to back, so the group's
 // weights are fetched once (rows that fit, 512 tokens: 0.5-0.9 % faster so).
 // Blocks past the work (padding, passes the sort did not fill) exit.
-template <bool DUAL, bool MLX>
+template <bool DUAL, bool MLX, bool NARROW>
 __device__ __attribute__((always_inline)) void pf_grid(const PfArgs& a, uint8_t* s_pf) {
   int b = blockIdx.x;
   const bool second = b >= a.n_items0;
@@ -549,17 +550,17 @@ __device__ __attribute__((always_inline)) void pf_grid(const PfArgs& a, uint8_t*
   }
   if (exact) {
     switch ((rows + 15) / 16) {
-      case 1: pf_item<DUAL, 1, false, MLX>(P, ng, row0, rows, e, ks, s_pf, a.f16_flag, a.flag_out); break;
-      case 2: pf_item<DUAL, 2, false, MLX>(P, ng, row0, rows, e, ks, s_pf, a.f16_flag, a.flag_out); break;
-      case 3: pf_item<DUAL, 3, false, MLX>(P, ng, row0, rows, e, ks, s_pf, a.f16_flag, a.flag_out); break;
-      default: pf_item<DUAL, 4, false, MLX>(P, ng, row0, rows, e, ks, s_pf, a.f16_flag, a.flag_out); break;
+      case 1: pf_item<DUAL, 1, false, MLX, NARROW>(P, ng, row0, rows, e, ks, s_pf, a.f16_flag, a.flag_out); break;
+      case 2: pf_item<DUAL, 2, false, MLX, NARROW>(P, ng, row0, rows, e, ks, s_pf, a.f16_flag, a.flag_out); break;
+      case 3: pf_item<DUAL, 3, false, MLX, NARROW>(P, ng, row0, rows, e, ks, s_pf, a.f16_flag, a.flag_out); break;
+      default: pf_item<DUAL, 4, false, MLX, NARROW>(P, ng, row0, rows, e, ks, s_pf, a.f16_flag, a.flag_out); break;
     }
   } else {
     switch ((rows + 15) / 16) {
-      case 1: pf_item<DUAL, 1, true, MLX>(P, ng, row0, rows, e, ks, s_pf, a.f16_flag, a.flag_out); break;
-      case 2: pf_item<DUAL, 2, true, MLX>(P, ng, row0, rows, e, ks, s_pf, a.f16_flag, a.flag_out); break;
-      case 3: pf_item<DUAL, 3, true, MLX>(P, ng, row0, rows, e, ks, s_pf, a.f16_flag, a.flag_out); break;
-      default: pf_item<DUAL, 4, true, MLX>(P, ng, row0, rows, e, ks, s_pf, a.f16_flag, a.flag_out); break;
+      case 1: pf_item<DUAL, 1, true, MLX, NARROW>(P, ng, row0, rows, e, ks, s_pf, a.f16_flag, a.flag_out); break;
+      case 2: pf_item<DUAL, 2, true, MLX, NARROW>(P, ng, row0, rows, e, ks, s_pf, a.f16_flag, a.flag_out); break;
+      case 3: pf_item<DUAL, 3, true, MLX, NARROW>(P, ng, row0, rows, e, ks, s_pf, a.f16_flag, a.flag_out); break;
+      default: pf_item<DUAL, 4, true, MLX, NARROW>(P, ng, row0, rows, e, ks, s_pf, a.f16_flag, a.flag_out); break;
     }
   }
 }
@@ -567,20 +568,29 @@ __device__ __attribute__((always_inline)) void pf_grid(const PfArgs& a, uint8_t*
 template <bool DUAL>
 __global__ __launch_bounds__(kPfThreads) void pf_gemm(PfArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t s_pf[];
-  pf_grid<DUAL, false>(a, s_pf);
+  pf_grid<DUAL, false, false>(a, s_pf);
 }
 
 // MLX-layout weights: the lane's word reads and row-map scatter take a few
 // registers more, which would leave two waves per SIMD; held to three
 __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(3))) void pf_gemm_mlx(PfArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t s_pf[];
-  pf_grid<false, true>(a, s_pf);
+  pf_grid<false, true, false>(a, s_pf);
+}
+
+// Narrow column groups for grids of few work items (PfSet::narrow): with a
+// wave or two per SIMD a unit takes as long as the wave's own chain of
+// dequantisation and products, which half the columns shorten (0.61 -> 0.46
+// us per unit at 32 rows; more units in flight, six stages, gave nothing).
+__global__ __launch_bounds__(kPfThreads) void pf_gemm_mlx_narrow(PfArgs a) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t s_pf[];
+  pf_grid<false, true, true>(a, s_pf);
 }
 
 }  // namespace
 
 int pf_items(PfSet& s, bool dual) {
-  const int per_group = kPfWaves * (dual ? pf_nb<true>() : pf_nb<false>());
+  const int per_group = kPfWaves * (dual || s.narrow ? 1 : pf_nb<false>());
   s.ng = (s.nt + per_group - 1) / per_group;
   if (s.pass_n)  // pass-major per XCD
     return kXcds * s.ng * ((s.max_pass + kXcds - 1) / kXcds);
@@ -611,7 +621,13 @@ hipError_t launch_pf(const PfArgs& a, bool dual, hipStream_t stream) {
   if (mlx && (dual || (a.n_items0 && !a.s0.mw) || (a.n_items1 && !a.s1.mw))) return hipErrorInvalidValue;
   for (const PfSet* s : {&a.s0, &a.s1})  // rounded outputs only
     if (mlx && (s->out32 || s->act || s->bias || s->res)) return hipErrorInvalidValue;
-  if (dual)
+  const bool narrow = a.n_items0 ? a.s0.narrow : a.s1.narrow;
+  if ((a.n_items0 && !a.s0.narrow == narrow) || (a.n_items1 && !a.s1.narrow == narrow) || (narrow && !mlx))
+    return hipErrorInvalidValue;
+  if (narrow)
+    hipLaunchKernelGGL(pf_gemm_mlx_narrow, dim3(n), dim3(kPfThreads), (kPfStages * pf_stage_bytes<false, true>()), stream,
+                       a);
+  else if (dual)
     hipLaunchKernelGGL(pf_gemm<true>, dim3(n), dim3(kPfThreads), pf_lds_bytes(true), stream, a);
   else if (mlx)
     hipLaunchKernelGGL(pf_gemm_mlx, dim3(n), dim3(kPfThreads), pf_lds_bytes(false), stream, a);
