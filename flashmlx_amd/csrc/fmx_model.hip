@@ -359,7 +359,7 @@ __global__ __launch_bounds__(256) void rope_cache_kernel(RopeArgs a) {
 //   out_d = bf16(num_d / den)
 // (one range: f_0 = 1, the range's own sums).
 //
-// Spread: with few (token, head) pairs and many keys (kAttnSpreadKeys, known
+// Spread: with few (token, head) pairs and many keys (attn_spread_keys, known
 // on the device only) one workgroup per pair leaves CUs idle and is bound by
 // what one CU draws (16 heads, 3500 keys: 1.8 MB each at 40 GB/s); the
 // launch then has Z workgroups per pair, which exit but for the first on a
@@ -376,8 +376,7 @@ __global__ __launch_bounds__(256) void rope_cache_kernel(RopeArgs a) {
 // sequence at 3500 keys: 45 -> 14 us per layer; a 4-layer step of one
 // sequence at 600 / 3500 keys 262 -> 236 / 367 -> 247 us, of 4 at 600 / 3500
 // 328 -> 322 / 439 -> 368, of 8 at 700 / 1500 / 3500 388 -> 385 / 417 -> 417
-// / 515 -> 487. From 512 keys on because every range is then a whole round
-// (at 400 keys and 24 layers the hand-over cost more than it saved).
+// / 515 -> 487.
 //
 // q and the new key are
 // rotated from the q/k/v row as rope_cache_kernel does; the new key and
@@ -425,14 +424,15 @@ __global__ __launch_bounds__(kWave * kAttnSplitMax) void attn_split_kernel(AttnA
   uint16_t* kb = a.kc + cbase;
   uint16_t* vb = a.vc + cbase;
   // spread over the Z workgroups, or all ranges on the first
+  constexpr int R = kAttnSplitMax / Z;
   bool spread = false;
+  const int zs = (S + R - 1) / R;  // workgroups with ranges
   if constexpr (Z > 1) {
-    spread = nk > kAttnSpreadKeys;
-    if (!spread && blockIdx.z) return;
+    spread = nk > attn_spread_keys(Z);
+    if (static_cast<int>(blockIdx.z) >= (spread ? zs : 1)) return;
   }
   // this wave's range; keys before jg come from the cache (p, the last key
   // of the last range, from LDS)
-  constexpr int R = kAttnSplitMax / Z;
   const int range = spread ? static_cast<int>(blockIdx.z) * R + wave / Z : wave;
   const bool active = range < S;
   const int j0 = active ? static_cast<int>(static_cast<int64_t>(nk) * range / S) : 0;
@@ -498,7 +498,7 @@ __global__ __launch_bounds__(kWave * kAttnSplitMax) void attn_split_kernel(AttnA
   };
   if (spread) {
     if (js < jg) load_keys(js);
-    if (vwave) load_spread(0, vv);
+    if (vwave && active) load_spread(0, vv);
   } else if (active && j0 < jg) {
     load_keys(j0);
     load_values(j0);
@@ -600,7 +600,7 @@ __global__ __launch_bounds__(kWave * kAttnSplitMax) void attn_split_kernel(AttnA
         s_e[jk - j0] = exp_det(static_cast<double>(s_s[jk - j0]) - static_cast<double>(m));
   }
   if (spread) {
-    if (vwave) load_spread(1, v2);
+    if (vwave && active) load_spread(1, v2);
     lds_barrier();  // (a __syncthreads would wait for the batches in flight)
   } else {
     __syncthreads();
@@ -670,7 +670,7 @@ __global__ __launch_bounds__(kWave * kAttnSplitMax) void attn_split_kernel(AttnA
       __syncthreads();
       if (tid == 0)
         s_last = __hip_atomic_fetch_add(a.arrived + t * a.nh + h, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
-                 static_cast<uint32_t>(Z - 1);
+                 static_cast<uint32_t>(zs - 1);
       // the new key and value into the caches
       if (blockIdx.z == 0 && h % rep == 0 && tid < a.hd) {
         kb[static_cast<int64_t>(p) * a.hd + tid] = s_knew[tid];
@@ -928,11 +928,11 @@ hipError_t launch_rope_cache(const RopeArgs& a, int T, hipStream_t stream) {
 // Workgroups per (token, head) of a single-token forward: as many as the
 // CUs hold at one workgroup each, when the cache is long enough for any.
 static int attn_spread_wgs(const AttnArgs& a, int T) {
-  if (!a.part || a.hd != kAttnSplitMaxHd || a.max_seq <= kAttnSpreadKeys) return 1;
+  if (!a.part || a.hd != kAttnSplitMaxHd) return 1;
   const int64_t pairs = static_cast<int64_t>(T) * a.nh;
   int z = 1;
   while (z < kAttnSplitMax && pairs * 2 * z <= kAttnSpreadWgs) z *= 2;
-  return z;
+  return a.max_seq > attn_spread_keys(z) ? z : 1;
 }
 
 hipError_t launch_attn(const AttnArgs& a, int T, hipStream_t stream) {

@@ -120,11 +120,16 @@ struct AttnArgs {
 constexpr int kAttnSplitMax = 16;
 constexpr int kAttnSplitKeys = 32;
 constexpr int kAttnSplitMaxHd = 128;
-// contexts of more keys than this are spread over several workgroups per
-// (token, head), as many (a power of two up to kAttnSplitMax) as keep the
-// grid within kAttnSpreadWgs
-constexpr int kAttnSpreadKeys = kAttnSplitMax * kAttnSplitKeys;
+// long contexts are spread over several workgroups per (token, head), as many
+// (z, a power of two up to kAttnSplitMax) as keep the grid within
+// kAttnSpreadWgs (one per CU: with 512, 2 and 4 sequences 6 us per layer
+// slower), from more keys than attn_spread_keys(z) on: what the hand-over
+// costs is earned sooner the fewer workgroups there are otherwise (4-layer
+// step, one workgroup -> spread: 1 sequence at 250 / 300 / 500 keys 223 ->
+// 223 / 226 -> 222 / 241 -> 225 us; 2 at 300 / 500 261 -> 262 / 274 -> 265; 4
+// at 300 / 500 288 -> 299 / 304 -> 308; 8 at 500 352 -> 355)
 constexpr int kAttnSpreadWgs = 256;
+__host__ __device__ constexpr int attn_spread_keys(int z) { return z >= 16 ? 256 : z == 8 ? 384 : 512; }
 // the longest range of a cache of max_seq positions
 __host__ __device__ inline int attn_split_range_keys(int64_t max_seq) {
   const int64_t r = (max_seq + kAttnSplitMax - 1) / kAttnSplitMax;

@@ -3,8 +3,9 @@ the same key ranges, sums and order as one workgroup forms, so a decode step
 of a few sequences (16 heads: 1, 2, 4 and 8 of them are spread over 16, 8, 4
 and 2 workgroups) has the bits of a step of 16, which is not spread and which
 test_gpu_attention.py pins to the oracle. Positions on both sides of the
-spread's threshold (512 keys), of whole 32-key rounds, with the new key in
-each key class, up to the longest cache; one key dominates some sequences."""
+spread's thresholds (256, 384, 512 keys) and of whole 32-key rounds, fewer than
+16 ranges among them, up to the longest cache; one key dominates some
+sequences."""
 from __future__ import annotations
 
 import numpy as np
@@ -15,7 +16,7 @@ from test_gpu_model import _build, _tiny_cfg
 
 pytestmark = pytest.mark.gpu
 
-POSITIONS = [511, 3499, 512, 4095, 513, 514, 515, 700, 1023, 1024, 1999, 2048, 2571, 3333, 4094, 1]
+POSITIONS = [511, 3499, 512, 4095, 255, 256, 257, 383, 384, 385, 300, 2048, 480, 3333, 1023, 1]
 
 
 @pytest.mark.parametrize("nkv", [16, 4])
