@@ -38,7 +38,8 @@ STAGE_OF = [
     (r"attn_split_kernel", "attention (single token)"),
     (r"attn_mfma_kernel|attn_kernel", "attention (several tokens)"),
     (r"dense_dec_kernel<true", "q/k/v with input norm"),
-    (r"dense_dec_kernel<false", "o_proj, lm_head"),
+    (r"dense_dec_kernel<false", "q/k/v, o_proj"),
+    (r"dense_wide_kernel", "lm_head"),
     (r"greedy_kernel", "argmax"),
     (r"rmsnorm_kernel", "norm"),
     # the Nemotron-H block's kernels
