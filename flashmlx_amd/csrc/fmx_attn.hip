@@ -3,10 +3,13 @@
 // rope_cache_kernel: causal, over the KV cache
 // (mx::fast::scaled_dot_product_attention, server/src/model.cpp:879-882).
 //
-//   attn_mfma_kernel  head sizes 64 and 128: tiles of query rows against
-//                     blocks of keys on the matrix cores
+//   attn_tile_kernel  head sizes 64 and 128: tiles of 16 query rows against
+//                     tiles of 16 keys on the matrix cores
 //   attn_kernel       other head sizes and the smallest calls: one workgroup
 //                     per (token, head)
+//
+// Both form the same sums in the same order, so a row has the same bits on
+// either.
 //
 // Single-token forwards: attn_split_kernel (fmx_model.hip).
 #include <algorithm>
@@ -32,6 +35,7 @@ namespace {
 constexpr int kAttnThreads = 256;
 constexpr int kAttnWaves = kAttnThreads / kWave;
 constexpr int kAttnBatch = 32;  // keys whose value words are loaded together
+constexpr int64_t kLdsBytes = 160 * 1024;  // per CU
 
 size_t attn_row_lds(int64_t max_seq) {
   return static_cast<size_t>(align_up(max_seq * 12, 8) + 8 * kAttnWaves * (kAttnMaxHd + 1) +
@@ -176,85 +180,107 @@ __global__ __launch_bounds__(kAttnThreads) void attn_kernel(AttnArgs a) {
   attn_row<PAIRS>(a, blockIdx.x, blockIdx.y, s_at);
 }
 
-// ------------------------------------------------------------------ MFMA tiles
+// ------------------------------------------------------------------ tiles
 
-// One workgroup per (64 / KW query rows of one sequence, q head): four waves
-// in groups of KW that share 16 rows, each wave with keys of its own (KW 1:
-// every wave its own 16 rows and all keys; KW 4: the waves' sums are added
-// at the end). Blocks of KB keys and values stream through a two-stage LDS
-// ring by LDS DMA, 16-byte chunks XOR-swizzled by row.
+// One workgroup per (16 query rows of one sequence, q head): the sums of
+// attn_row, bit for bit, on the matrix cores, whose fp32 and fp64 products
+// over K = 4 add their terms one after the other, each a fused multiply-add
+// (measured against fma chains, subnormal results among them):
+//   scores S^T = K Q^T by v_mfma_f32_16x16x4_f32, dimensions in order, then
+//     times scale;
+//   weights by exp_det's steps;
+//   sums O^T += V^T P^T by v_mfma_f64_16x16x4_f64, keys in order, den by
+//     v_mfma_f64_4x4x4_4b_f64 with ones.
+// Wave w has quarter w of the keys, as in attn_row. The rows' quarters begin
+// up to 12 keys apart: the wave runs over the keys of any of its rows, and
+// the weight of a key outside a row's own quarter is 0, which leaves the
+// row's sums as they are.
 //
-// Scores come out transposed, S^T = K Q^T (v_mfma_f32_16x16x32_bf16, exact
-// products, fp32 sums): lane (i16, j) holds query i16 against keys 4j + r of
-// each 16-key tile, which is the B operand of O^T = V^T P^T as it stands;
-// V^T comes from the row-major values by the transposing LDS read
-// (ds_read_b64_tr_b16: 4 keys x 16 dimensions per 16 lanes).
+// The weights need the row's largest score first. A pass of bf16 products
+// (v_mfma_f32_16x16x32_bf16, an eighth of the score steps' time) finds the
+// key that has it, whose score is then formed like all others; the second
+// pass checks that no score is larger, and the tile is done again behind a
+// pass of fp32 scores where one is (a near tie that the bf16 products' order
+// of summation decided otherwise).
 //
-// The softmax weights keep their 24 bits: p = hi + mid + lo, three bf16
-// values cut from its fp32 pattern, three MFMAs. fp32 sums run over at most
-// kFoldKeys keys and are then added to fp64 sums (as the row kernel's), one
-// division and one rounding at the end. The running maximum moves only when
-// a score exceeds it by more than 2^8 in weight, which the sums have the
-// range for.
+// Row 4j + r of a 16-key score tile is key 4r + j, so lane (i16, j) ends up
+// with query i16 and key 4r + j in register r: the B operand of step r of the
+// value products as it stands. Nothing passes through LDS but the maxima and
+// the quarter sums at the end: a lane loads 16 bytes of a key (chunk 4i + j
+// of its 8-dimension chunks), pairs dimensions d and d + 4 and exchanges the
+// pairs with the three other lanes of the key (4 x 4 transposes by
+// v_permlane32_swap and v_permlane16_swap), which leaves it dimension 4s + j
+// of every step s. Values: DT dimensions DT i16 + dt of a key per lane, so
+// row i16 of dimension tile dt.
 //
 // A row that is not finite at the end (inf or NaN in the keys or values its
-// tile read, those beyond its own position included, or an overflow of the
-// fp32 sums) is computed again by attn_row.
+// tile read, those beyond its own position included) is computed again by
+// attn_row.
 //
-// Bound: per 16 rows x 64 keys x 128 dimensions a wave issues 64 MFMAs (48
-// of them the weights' three parts) and about 200 VALU instructions, on two
-// waves per SIMD (241 VGPRs, half of a CU's LDS per workgroup). 16 heads of
-// 128, one sequence of 3001 tokens: 113 us (18.4 GFLOP causal, 3750 us as
-// rows), 1024 tokens 37 us (519), 512 tokens behind 1024 cached ones 47 us
-// (570).
-constexpr int kFoldKeys = 256;
-constexpr float kMaxSlack = 8.0f;
+// Bound by the matrix cores' fp64 and fp32 rates (58 and 155 TFLOP/s,
+// measured): one sequence of 3001 tokens, 16 heads of 128, 18.4 GFLOP of
+// each, 433 us, took 737 us (the row kernel 3300); the difference are the
+// exps (75 us), the operands' preparation (3 VALU instructions per score
+// step, which do not overlap with the fp32 products) and the loads. With
+// the first pass in fp32 870 us. 1024 tokens 119 us (495 as rows), 512 tokens
+// behind 1024 cached ones 138 us (552). Two tiles at a time, or the next
+// tile's score steps between the value products, gave nothing: with two waves
+// per SIMD the chains are covered.
+constexpr int kTileRows = 16;
 
-typedef short i16x4_t __attribute__((ext_vector_type(4)));
+// exp_det of r <= 0 or NaN without branches, so that several run side by
+// side (r > 0: some value)
+__device__ inline double exp_neg(double r) {
+  const double e = exp_steps(r, fmax(rint(r * kExpLog2e), -1000.0));
+  return r < -690.0 ? 0.0 : e;
+}
 
-template <int HD, int KW>
-struct AttnTile {
-  static constexpr int kRows = 64 / KW;              // query rows per workgroup
-  static constexpr int kKeysWave = KW == 1 ? 64 : 32;  // keys per wave and block
-  static constexpr int kKeys = kKeysWave * KW;       // keys per block
-  static constexpr int kStage = kKeys * HD * 2 * 2;  // a block's keys and values
-  static constexpr int kMerge = KW == 1 ? 0 : KW * 16 * (HD + 2) * 8;
-  static constexpr int kLds = 2 * kStage > kMerge ? 2 * kStage : kMerge;
-};
+typedef double f64x4_t __attribute__((ext_vector_type(4)));
 
 template <int HD>
-__device__ inline bf16x8_t attn_vt(const uint8_t* sv, int key, int dt, int i16, int j) {
-  // dimensions 16 dt + i16 of keys key + 4 j + (0..3) and key + 16 + 4 j + (0..3)
-  constexpr int CH = HD / 8;
-  union {
-    i16x4_t h[2];
-    bf16x8_t v;
-  } u;
+struct AttnTile {
+  static constexpr int NI = HD / 32;       // 16-byte loads of a lane per key tile
+  static constexpr int NC = HD / 8;        // 8-dimension chunks: two score steps each
+  static constexpr int DT = HD / 16;       // 16-dimension tiles
+  static constexpr int kRow = HD + 2;      // doubles of a row's sums: dimensions, den, (padding)
+  static constexpr int kLds = kAttnWaves * kTileRows * kRow * 8;
+};
+
+// Raw chunks 4i + j of a row to its dimension pairs (8c + j, 8c + 4 + j),
+// c = 0 .. NC - 1, j = lane / 16.
+template <int NI>
+__device__ inline void attn_pairs(const u32x4_t (&raw)[NI], uint32_t (&pr)[4 * NI]) {
 #pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    const int row = key + 16 * t + 4 * j + (i16 >> 2);
-    const uint8_t* p = sv + row * (HD * 2) + (((2 * dt + ((i16 >> 1) & 1)) ^ (2 * (row & (CH / 2 - 1)))) << 4) +
-                       (i16 & 1) * 8;
-    u.h[t] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4_t*)p);
+  for (int i = 0; i < NI; ++i) {
+    // bytes 0, 1 of the first word below, bytes 4, 5: 2, 3 of the second
+    uint32_t r0 = __builtin_amdgcn_perm(raw[i][2], raw[i][0], 0x05040100u);
+    uint32_t r1 = __builtin_amdgcn_perm(raw[i][2], raw[i][0], 0x07060302u);
+    uint32_t r2 = __builtin_amdgcn_perm(raw[i][3], raw[i][1], 0x05040100u);
+    uint32_t r3 = __builtin_amdgcn_perm(raw[i][3], raw[i][1], 0x07060302u);
+    const auto a = __builtin_amdgcn_permlane32_swap(r0, r2, false, false);
+    const auto b = __builtin_amdgcn_permlane32_swap(r1, r3, false, false);
+    const auto c = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false);
+    const auto d = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
+    pr[4 * i] = c[0];
+    pr[4 * i + 1] = c[1];
+    pr[4 * i + 2] = d[0];
+    pr[4 * i + 3] = d[1];
   }
-  return u.v;
 }
 
-// words holding the high halves of two fp32 patterns
-__device__ inline uint32_t high_halves(float lo, float hi) {
-  return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
-}
+__device__ inline float pair_lo(uint32_t w) { return __uint_as_float(w << 16); }
+__device__ inline float pair_hi(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
 
-template <int HD, int KW>
-__global__ __launch_bounds__(kAttnThreads) __attribute__((amdgpu_waves_per_eu(KW == 1 ? 2 : 1)))
-void attn_mfma_kernel(AttnArgs a, int B, int n_tiles) {
-  using T = AttnTile<HD, KW>;
-  constexpr int CH = HD / 8, RB = HD * 2, NQ = HD / 32, ND = HD / 16, NT = T::kKeysWave / 16;
-  constexpr int RPP = 1024 / RB;                       // rows per 1 KB LDS DMA piece
-  constexpr int PW = T::kKeys / RPP / kAttnWaves;      // pieces per wave, of keys and of values
-  constexpr int kFold = kFoldKeys / T::kKeysWave;      // blocks between folds
+template <int HD>
+__global__ __launch_bounds__(kAttnThreads) __attribute__((amdgpu_waves_per_eu(2)))
+void attn_tile_kernel(AttnArgs a, int B, int n_tiles) {
+  using T = AttnTile<HD>;
+  constexpr int NI = T::NI, NC = T::NC, DT = T::DT;
   extern __shared__ __attribute__((aligned(16))) uint8_t s_at[];
-  __shared__ uint32_t s_bad[T::kRows];
+  __shared__ uint32_t s_bad[kTileRows];
+  __shared__ float s_max[kAttnWaves][kTileRows];
+  __shared__ int s_key[kAttnWaves][kTileRows];
+  __shared__ uint32_t s_over[kAttnWaves];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -268,263 +294,257 @@ void attn_mfma_kernel(AttnArgs a, int B, int n_tiles) {
   const int bh = static_cast<int>(blockIdx.x) % nhb;
   const int b = bh / a.nh, hi = bh - b * a.nh;
   const int g = hi % a.nkv, h = g * (a.nh / a.nkv) + hi / a.nkv;
-  const int l0 = tile * T::kRows;
-  const int lw = l0 + (KW == 1 ? 16 * wave : 0);
-  const int l = min(lw + i16, a.L - 1);                // rows past the sequence repeat its last
+  const int l0 = tile * kTileRows;
+  const int l = min(l0 + i16, a.L - 1);  // rows past the sequence repeat its last
   const int p = token_pos(a.offs, a.off, b, l, a.max_seq);
-  const int p_lo = token_pos(a.offs, a.off, b, min(lw, a.L - 1), a.max_seq);
-  const int p_wave = token_pos(a.offs, a.off, b, min(lw + 15, a.L - 1), a.max_seq);
-  const int p_hi = token_pos(a.offs, a.off, b, min(l0 + T::kRows - 1, a.L - 1), a.max_seq);
+  const int p_lo = token_pos(a.offs, a.off, b, l0, a.max_seq);
+  const int p_hi = token_pos(a.offs, a.off, b, min(l0 + kTileRows - 1, a.L - 1), a.max_seq);
   const int64_t cbase = (cache_slot(a.slots, a.n_slots, b) * a.nkv + g) * a.max_seq * HD;
   const uint16_t* kb = a.kc + cbase;
   const uint16_t* vb = a.vc + cbase;
 
-  // the wave's 16 rotated query rows, B operands
-  bf16x8_t Q[NQ];
-  const uint16_t* qrow = a.q + ((static_cast<int64_t>(b) * a.L + l) * a.nh + h) * HD + 8 * j;
+  auto load_key = [&](u32x4_t (&raw)[NI], int key) {
+    const uint16_t* src = kb + static_cast<int64_t>(key) * HD + 8 * j;
 #pragma unroll
-  for (int q = 0; q < NQ; ++q) Q[q] = *reinterpret_cast<const bf16x8_t*>(qrow + 32 * q);
-
-  auto issue = [&](int key0, uint8_t* st) {
+    for (int i = 0; i < NI; ++i) raw[i] = *reinterpret_cast<const u32x4_t*>(src + 32 * i);
+  };
+  // keys key0 .. key0 + 15 (past the last key: that key again)
+  const int krow = 4 * (i16 & 3) + (i16 >> 2);
+  auto load_keys = [&](u32x4_t (&raw)[NI], int key0) { load_key(raw, min(key0 + krow, p_hi)); };
+  uint32_t vw[4][DT / 2];
+  auto load_values = [&](int key0) {
 #pragma unroll
-    for (int pc = 0; pc < PW; ++pc) {
-      const int piece = pc * kAttnWaves + wave;
-      const int row = piece * RPP + lane / CH, c = lane % CH;
-      const int64_t src = static_cast<int64_t>(min(key0 + row, p_hi)) * HD;  // past the last key: that key again
-      __builtin_amdgcn_global_load_lds(static_cast<const void*>(kb + src + 8 * (c ^ (row & (CH - 1)))),
-                                       (__attribute__((address_space(3))) void*)(st + piece * 1024), 16, 0, 0);
-      __builtin_amdgcn_global_load_lds(static_cast<const void*>(vb + src + 8 * (c ^ (2 * (row & (CH / 2 - 1))))),
-                                       (__attribute__((address_space(3))) void*)(st + T::kStage / 2 + piece * 1024),
-                                       16, 0, 0);
+    for (int r = 0; r < 4; ++r) {
+      const uint16_t* src = vb + static_cast<int64_t>(min(key0 + 4 * r + j, p_hi)) * HD + DT * i16;
+      if constexpr (DT == 8) {
+        const u32x4_t w = *reinterpret_cast<const u32x4_t*>(src);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) vw[r][q] = w[q];
+      } else {
+        const u32x2_t w = *reinterpret_cast<const u32x2_t*>(src);
+#pragma unroll
+        for (int q = 0; q < 2; ++q) vw[r][q] = w[q];
+      }
     }
   };
 
-  f32x4_t acc[ND];
-  double o[ND][4], den = 0.0;
-  float m = -__builtin_huge_valf();
+  u32x4_t raw[NI], qr[NI];
+  load_keys(raw, wave * 16);
+  const uint16_t* qrow = a.q + ((static_cast<int64_t>(b) * a.L + l) * a.nh + h) * HD + 8 * j;
 #pragma unroll
-  for (int d = 0; d < ND; ++d) {
-    acc[d] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int i = 0; i < NI; ++i) qr[i] = *reinterpret_cast<const u32x4_t*>(qrow + 32 * i);
+  float Q[2 * NC];  // query i16, dimensions 4s + j
+  {
+    uint32_t qp[4 * NI];
+    attn_pairs<NI>(qr, qp);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) o[d][r] = 0.0;
-  }
-  // scores in units of log 2: the weights are powers of two
-  const float cs = a.scale * 1.4426950408889634f;
-  const int nb = p_hi / T::kKeys + 1;
-  const int kw = KW == 1 ? 0 : wave * T::kKeysWave;  // the wave's keys within a block
-  issue(0, s_at);
-  for (int blk = 0; blk < nb; ++blk) {
-    // this wave's pieces of the block have landed; behind the barrier every
-    // wave's have, and every wave's reads of the other stage are done
-    wait_vmcnt0();
-    lds_barrier();
-    if (blk + 1 < nb) issue((blk + 1) * T::kKeys, s_at + ((blk + 1) & 1) * T::kStage);
-    const uint8_t* sk = s_at + (blk & 1) * T::kStage;
-    const uint8_t* sv = sk + T::kStage / 2;
-    const int key0 = blk * T::kKeys + kw;
-    if (key0 <= p_wave) {
-      f32x4_t S[NT];
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) {
-        S[nt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-        const int row = kw + 16 * nt + i16;
-#pragma unroll
-        for (int q = 0; q < NQ; ++q)
-          S[nt] = mfma_bf16(*reinterpret_cast<const bf16x8_t*>(sk + row * RB + (((4 * q + j) ^ (row & (CH - 1))) << 4)),
-                            Q[q], S[nt]);
-      }
-      const bool diag = key0 + T::kKeysWave - 1 > p_lo;
-      float mx = -__builtin_huge_valf();
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const float x = S[nt][r] * cs;
-          mx = fmaxf(mx, diag && key0 + 16 * nt + 4 * j + r > p ? -__builtin_huge_valf() : x);
-        }
-      if (__ballot(mx > m + kMaxSlack)) {
-        mx = fmaxf(mx, __shfl_xor(mx, 16));
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
-        const float mn = fmaxf(m, mx);
-        // the same factor on both sums, so its rounding cancels
-        const float f = mn == m ? 1.0f : __builtin_amdgcn_exp2f(m - mn);
-        m = mn;
-        den *= static_cast<double>(f);
-#pragma unroll
-        for (int d = 0; d < ND; ++d)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            acc[d][r] *= f;
-            o[d][r] *= static_cast<double>(f);
-          }
-      }
-      float ds = 0.0f;
-      u32x4_t P[NT / 2][3];
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) {
-        float w[4], w2[4], w3[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          w[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(S[nt][r], cs, -m));
-          if (diag && key0 + 16 * nt + 4 * j + r > p) w[r] = 0.0f;
-          ds += w[r];
-          w2[r] = w[r] - __uint_as_float(__float_as_uint(w[r]) & 0xffff0000u);
-          w3[r] = w2[r] - __uint_as_float(__float_as_uint(w2[r]) & 0xffff0000u);
-        }
-#pragma unroll
-        for (int c = 0; c < 2; ++c) {
-          P[nt / 2][0][2 * (nt & 1) + c] = high_halves(w[2 * c], w[2 * c + 1]);
-          P[nt / 2][1][2 * (nt & 1) + c] = high_halves(w2[2 * c], w2[2 * c + 1]);
-          P[nt / 2][2][2 * (nt & 1) + c] = high_halves(w3[2 * c], w3[2 * c + 1]);
-        }
-      }
-      den += static_cast<double>(ds);
-#pragma unroll
-      for (int ks = 0; ks < NT / 2; ++ks)
-#pragma unroll
-        for (int d = 0; d < ND; ++d) {
-          const bf16x8_t V = attn_vt<HD>(sv, kw + 32 * ks, d, i16, j);
-#pragma unroll
-          for (int c = 2; c >= 0; --c) acc[d] = mfma_bf16(V, __builtin_bit_cast(bf16x8_t, P[ks][c]), acc[d]);
-        }
-    }
-    if (blk % kFold == kFold - 1 || blk == nb - 1) {
-#pragma unroll
-      for (int d = 0; d < ND; ++d) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) o[d][r] += static_cast<double>(acc[d][r]);
-        acc[d] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-      }
+    for (int c = 0; c < NC; ++c) {
+      Q[2 * c] = pair_lo(qp[c]);
+      Q[2 * c + 1] = pair_hi(qp[c]);
     }
   }
-  den += __shfl_xor(den, 16);
-  den += __shfl_xor(den, 32);
+  auto scores = [&](const u32x4_t (&r)[NI]) {
+    uint32_t kp[4 * NI];
+    attn_pairs<NI>(r, kp);
+    f32x4_t S = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      S = __builtin_amdgcn_mfma_f32_16x16x4f32(pair_lo(kp[c]), Q[2 * c], S, 0, 0, 0);
+      S = __builtin_amdgcn_mfma_f32_16x16x4f32(pair_hi(kp[c]), Q[2 * c + 1], S, 0, 0, 0);
+    }
+    return S;
+  };
 
-  bool ovf = false;
-  if constexpr (KW == 1) {
-    // lane (i16, j): row i16, dimensions 16 d + 4 j + r
-    const double inv = 1.0 / den;
-    bool bad = !(den < __builtin_huge_val());
+  // this wave's quarter: row i16's keys [j0, j1), any row's [k_lo, k_hi),
+  // every row's [full_lo, full_hi)
+  const int quarter = (p + kAttnWaves) / kAttnWaves;
+  const int j0 = min(wave * quarter, p + 1), j1 = min(j0 + quarter, p + 1);
+  auto row_min = [](int v) {
 #pragma unroll
-    for (int d = 0; d < ND; ++d)
+    for (int o = 8; o >= 1; o >>= 1) v = min(v, __shfl_xor(v, o));
+    return __builtin_amdgcn_readfirstlane(v);
+  };
+  const int k_lo = row_min(j0), k_hi = -row_min(-j1);
+  const int full_lo = -row_min(-j0), full_hi = row_min(j1);
+
+  double* s_o = reinterpret_cast<double*>(s_at);
+  for (bool exact = false;; exact = true) {
+    // 1. each row's largest score; the waves take every fourth key tile
+    float m = -__builtin_huge_valf();
+    if (!exact) {
+      // that of the key whose bf16 products sum up largest
+      int mk = 0;
+      for (int key0 = wave * 16; key0 <= p_hi; key0 += 16 * kAttnWaves) {
+        f32x4_t S = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int r = 0; r < 4; ++r) bad |= !(fabs(o[d][r]) < __builtin_huge_val());
-    const uint64_t bm = __ballot(bad) >> i16;
-    bad = (bm & 0x0001000100010001ull) != 0;
-    if (j == 0) s_bad[16 * wave + i16] = bad && lw + i16 < a.L;
-    const bool store = !bad && lw + i16 < a.L;
-    const int64_t ob = (static_cast<int64_t>(b) * a.L + l) * a.ldo + static_cast<int64_t>(h) * HD;
+        for (int i = 0; i < NI; ++i)
+          S = mfma_bf16(__builtin_bit_cast(bf16x8_t, raw[i]), __builtin_bit_cast(bf16x8_t, qr[i]), S);
+        load_keys(raw, key0 + 16 * kAttnWaves);
 #pragma unroll
-    for (int d = 0; d < ND; ++d) {
-      uint16_t v[4], vh[4];
+        for (int r = 0; r < 4; ++r) {
+          const int key = key0 + 4 * r + j;
+          const bool up = S[r] > m && key <= p;
+          m = up ? S[r] : m;
+          mk = up ? key : mk;
+        }
+      }
+#pragma unroll
+      for (int o = 16; o <= 32; o *= 2) {
+        const float om = __shfl_xor(m, o);
+        const int ok = __shfl_xor(mk, o);
+        mk = om > m ? ok : mk;
+        m = fmaxf(m, om);
+      }
+      if (j == 0) {
+        s_max[wave][i16] = m;
+        s_key[wave][i16] = mk;
+      }
+      lds_barrier();
+      m = s_max[0][i16];
+      mk = s_key[0][i16];
+#pragma unroll
+      for (int w = 1; w < kAttnWaves; ++w) {
+        mk = s_max[w][i16] > m ? s_key[w][i16] : mk;
+        m = fmaxf(m, s_max[w][i16]);
+      }
+      // a tile of the rows' keys: row i16's score is on its diagonal
+      load_key(raw, mk);
+      const f32x4_t S = scores(raw);
+      m = i16 >> 2 == j ? (i16 & 2 ? (i16 & 1 ? S[3] : S[2]) : (i16 & 1 ? S[1] : S[0])) * a.scale
+                        : -__builtin_huge_valf();
+      m = fmaxf(m, __shfl_xor(m, 16));
+      m = fmaxf(m, __shfl_xor(m, 32));
+    } else {
+      for (int key0 = wave * 16; key0 <= p_hi; key0 += 16 * kAttnWaves) {
+        load_keys(raw, key0);
+        const f32x4_t S = scores(raw);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) m = fmaxf(m, key0 + 4 * r + j > p ? -__builtin_huge_valf() : S[r] * a.scale);
+      }
+      m = fmaxf(m, __shfl_xor(m, 16));
+      m = fmaxf(m, __shfl_xor(m, 32));
+      if (j == 0) s_max[wave][i16] = m;
+      lds_barrier();
+#pragma unroll
+      for (int w = 0; w < kAttnWaves; ++w) m = fmaxf(m, s_max[w][i16]);
+    }
+
+    // 2. the wave's quarter
+    load_keys(raw, k_lo);
+    load_values(k_lo);
+    const double md = static_cast<double>(m);
+    float seen = m;
+    f64x4_t acc[DT];
+    double den = 0.0;
+#pragma unroll
+    for (int d = 0; d < DT; ++d) acc[d] = f64x4_t{0.0, 0.0, 0.0, 0.0};
+    for (int key0 = k_lo; key0 < k_hi; key0 += 16) {
+      f32x4_t S = scores(raw);
+      load_keys(raw, key0 + 16);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) S[r] *= a.scale;
+      double e[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) e[r] = exp_neg(static_cast<double>(S[r]) - md);
+      if (key0 < full_lo || key0 + 16 > full_hi) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int key = key0 + 4 * r + j;
+          const bool own = key >= j0 && key < j1;
+          e[r] = own ? e[r] : 0.0;
+          S[r] = own ? S[r] : m;
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) seen = fmaxf(seen, S[r]);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        v[r] = f64_to_bf16(o[d][r] * inv);
-        ovf |= store && bf16_f16_overflow(v[r]);
-        vh[r] = static_cast<uint16_t>(bf16_to_f16_bits(v[r]));
+        den = __builtin_amdgcn_mfma_f64_4x4x4f64(1.0, e[r], den, 0, 0, 0);
+#pragma unroll
+        for (int d = 0; d < DT; ++d) {
+          const uint32_t w = vw[r][d / 2];
+          acc[d] = __builtin_amdgcn_mfma_f64_16x16x4f64(static_cast<double>(d & 1 ? pair_hi(w) : pair_lo(w)), e[r],
+                                                        acc[d], 0, 0, 0);
+        }
       }
-      // P8 words pair element e with e + 4: the lane with the chunk's
-      // elements 0..3 writes words 0 and 1, its neighbour 2 and 3
-      const bool up = j & 1;
-      const uint32_t give = up ? vh[0] | (vh[1] << 16) : vh[2] | (vh[3] << 16);
-      const uint32_t got = __shfl_xor(give, 16);
-      const u32x2_t wh = up ? u32x2_t{(got & 0xffffu) | (static_cast<uint32_t>(vh[2]) << 16),
-                                      (got >> 16) | (static_cast<uint32_t>(vh[3]) << 16)}
-                            : u32x2_t{vh[0] | (got << 16), vh[1] | (got & 0xffff0000u)};
-      if (store) {
-        *reinterpret_cast<u32x2_t*>(a.out + ob + 16 * d + 4 * j) =
-            u32x2_t{v[0] | (static_cast<uint32_t>(v[1]) << 16), v[2] | (static_cast<uint32_t>(v[3]) << 16)};
-        if (a.outh) *reinterpret_cast<u32x2_t*>(a.outh + ob + 16 * d + 4 * j) = wh;
-      }
+      load_values(key0 + 16);
     }
-  } else {
-    // the waves' sums through LDS; thread (row, c): dimensions 8c .. 8c + 7
-    double* s_o = reinterpret_cast<double*>(s_at);
-    __syncthreads();  // the last block's reads
-    double* mine = s_o + (wave * 16 + i16) * (HD + 2);
+    double* mine = s_o + (wave * kTileRows + i16) * T::kRow;
 #pragma unroll
-    for (int d = 0; d < ND; ++d)
+    for (int r = 0; r < 4; ++r)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) mine[16 * d + 4 * j + r] = o[d][r];
-    if (j == 0) {
-      mine[HD] = den;
-      mine[HD + 1] = static_cast<double>(m);
-    }
-    __syncthreads();
-    const int row = tid >> 4, c = tid & 15;
-    double M = -__builtin_huge_val(), n[8], dn = 0.0;
+      for (int d = 0; d < DT; ++d) mine[DT * (j + 4 * r) + d] = acc[d][r];
+    if (j == 0) mine[HD] = den;
+    const bool over = __ballot(seen > m) != 0;
+    if (lane == 0) s_over[wave] = over;
+    lds_barrier();
+    if (exact || !(s_over[0] | s_over[1] | s_over[2] | s_over[3])) break;
+  }
+
+  // 3. the quarter sums, added in order; thread (row, c): dimensions 8c .. 8c + 7
+  const int row = tid >> 4, c = tid & 15;
+  const double* s = s_o + row * T::kRow;
+  constexpr int W = kTileRows * T::kRow;
+  const double dn = ((s[HD] + s[W + HD]) + s[2 * W + HD]) + s[3 * W + HD];
+  double n[8];
+  bool bad = !(dn < __builtin_huge_val());
 #pragma unroll
-    for (int e = 0; e < 8; ++e) n[e] = 0.0;
+  for (int e = 0; e < 8; ++e) {
+    const int d = min(8 * c, HD - 8) + e;
+    n[e] = ((s[d] + s[W + d]) + s[2 * W + d]) + s[3 * W + d];
+    bad |= !(fabs(n[e]) < __builtin_huge_val());
+  }
+  bad = ((__ballot(bad) >> (lane & 48)) & 0xffffull) != 0;
+  if (c == 0) s_bad[row] = bad && l0 + row < a.L;
+  bool ovf = false;
+  if (!bad && l0 + row < a.L && c < NC) {
+    const int64_t ob = (static_cast<int64_t>(b) * a.L + l0 + row) * a.ldo + static_cast<int64_t>(h) * HD + 8 * c;
+    u32x4_t v;
 #pragma unroll
-    for (int w = 0; w < KW; ++w) M = fmax(M, s_o[(w * 16 + row) * (HD + 2) + HD + 1]);
-#pragma unroll
-    for (int w = 0; w < KW; ++w) {
-      const double* s = s_o + (w * 16 + row) * (HD + 2);
-      // a wave without keys for the row: m = -inf, f = 0
-      const double f = static_cast<double>(__builtin_amdgcn_exp2f(static_cast<float>(s[HD + 1] - M)));
-      dn = __builtin_fma(s[HD], f, dn);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) n[e] = __builtin_fma(s[min(8 * c, HD - 8) + e], f, n[e]);
-    }
-    bool bad = !(dn < __builtin_huge_val());
-#pragma unroll
-    for (int e = 0; e < 8; ++e) bad |= !(fabs(n[e]) < __builtin_huge_val());
-    bad = ((__ballot(bad) >> (lane & 48)) & 0xffffull) != 0;
-    if (c == 0) s_bad[row] = bad && l0 + row < a.L;
-    if (!bad && l0 + row < a.L && c < CH) {
-      const double inv = 1.0 / dn;
-      const int64_t ob = (static_cast<int64_t>(b) * a.L + l0 + row) * a.ldo + static_cast<int64_t>(h) * HD + 8 * c;
-      u32x4_t v;
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        v[e] = f64_to_bf16(n[2 * e] * inv) | (static_cast<uint32_t>(f64_to_bf16(n[2 * e + 1] * inv)) << 16);
-      *reinterpret_cast<u32x4_t*>(a.out + ob) = v;
-      if (a.outh) *reinterpret_cast<u32x4_t*>(a.outh + ob) = bf16_chunk_to_f16_p8(v, ovf);
-    }
+    for (int e = 0; e < 4; ++e)
+      v[e] = f64_to_bf16(n[2 * e] / dn) | (static_cast<uint32_t>(f64_to_bf16(n[2 * e + 1] / dn)) << 16);
+    *reinterpret_cast<u32x4_t*>(a.out + ob) = v;
+    if (a.outh) *reinterpret_cast<u32x4_t*>(a.outh + ob) = bf16_chunk_to_f16_p8(v, ovf);
   }
   if (a.outh && __ballot(ovf) && lane == 0) atomicOr(a.flag, 1u);
 
   __syncthreads();
-  for (int r = 0; r < T::kRows; ++r)
+  for (int r = 0; r < kTileRows; ++r)
     if (s_bad[r]) {
       attn_row<1>(a, b * a.L + l0 + r, h, s_at);
       __syncthreads();
     }
 }
 
-template <int HD, int KW>
-hipError_t launch_mfma(const AttnArgs& a, int B, hipStream_t stream) {
-  using T = AttnTile<HD, KW>;
-  const int n_tiles = (a.L + T::kRows - 1) / T::kRows;
-  const size_t lds = std::max<size_t>(T::kLds, attn_row_lds(a.max_seq));
-  hipLaunchKernelGGL((attn_mfma_kernel<HD, KW>), dim3(n_tiles * a.nh * B), dim3(kAttnThreads), lds, stream, a, B,
-                     n_tiles);
+template <int HD>
+hipError_t launch_tiles(const AttnArgs& a, int B, hipStream_t stream) {
+  const int n_tiles = (a.L + kTileRows - 1) / kTileRows;
+  const size_t lds = std::max<size_t>(AttnTile<HD>::kLds, attn_row_lds(a.max_seq));
+  hipLaunchKernelGGL((attn_tile_kernel<HD>), dim3(n_tiles * a.nh * B), dim3(kAttnThreads), lds, stream, a, B, n_tiles);
   return hipGetLastError();
 }
 
 }  // namespace
 
-constexpr int64_t kRowsMax = 512;
-constexpr int kRowsMaxKeys = 64;
-constexpr int64_t kWideTiles = 128;
-
 hipError_t launch_attn_prefill(const AttnArgs& a, int T, hipStream_t stream) {
   if (T == 0) return hipSuccess;
   const int B = T / a.L;
   if (a.hd == 64 || a.hd == 128) {
-    // Few rows over few keys run as rows: a tile's fixed part (its code,
-    // the merge of the waves' sums) is then most of its time (24 tokens x 16
-    // heads 5.8 us as rows, 8.7 as tiles; 64 x 16 already 12.4 and 9.2).
-    // 64-row tiles from half a chip of them; below that 16-row tiles with
-    // the keys over the four waves (400 tokens x 16 heads, 112 tiles of 64:
-    // 20.4 us against 22.2; 512, 128 tiles: 22.8 / 23.7; 700, 176 tiles:
-    // 35.6 / 28.8; 100 tokens behind 1400: 25.9 / 45.4).
-    const bool rows = static_cast<int64_t>(T) * a.nh <= kRowsMax && !a.offs && a.off + a.L <= kRowsMaxKeys;
-    const bool wide = static_cast<int64_t>((a.L + 63) / 64) * a.nh * B >= kWideTiles;
-    if (!rows) {
-      if (a.hd == 128) return wide ? launch_mfma<128, 1>(a, B, stream) : launch_mfma<128, 4>(a, B, stream);
-      return wide ? launch_mfma<64, 1>(a, B, stream) : launch_mfma<64, 4>(a, B, stream);
-    }
+    // Few rows run as rows: a tile's four waves walk a quarter of the keys
+    // each, a row has four waves of its own. The line is where the row
+    // kernel's workgroups no longer run at the same time (three per CU by
+    // registers, fewer by LDS), for head size 64, whose tiles take 0.6 of the
+    // time, a third of that (us, rows / tiles, at keys 0 / 256 / 1024 / 3000
+    // before the call: 32 tokens x 16 heads of 128 7 / 14, 19 / 26, 48 / 59,
+    // 119 / 143; 48 x 16 8 / 15, 22 / 26, 62 / 60, 161 / 146; 64 x 16 13 / 15,
+    // 31 / 26, 82 / 60, 206 / 146; heads of 64, 8 x 16 6 / 10, 13 / 16, 32 /
+    // 36, 78 / 85; 24 x 16 7 / 10, 16 / 16, 43 / 36, 108 / 87). A little
+    // beyond it rows are still faster over few keys.
+    const int64_t n = static_cast<int64_t>(T) * a.nh;
+    const int64_t resident = 256 * std::min<int64_t>(3, kLdsBytes / attn_row_lds(a.max_seq));
+    const int64_t keys = a.offs ? a.max_seq : a.off + a.L;
+    const bool rows = n <= (a.hd == 128 ? resident : resident / 3) || (a.hd == 128 && n <= 1024 && keys <= 128);
+    if (!rows) return a.hd == 128 ? launch_tiles<128>(a, B, stream) : launch_tiles<64>(a, B, stream);
   }
   const dim3 grid(T, a.nh);
   const size_t lds = attn_row_lds(a.max_seq);

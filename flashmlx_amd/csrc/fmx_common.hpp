@@ -50,14 +50,10 @@ __device__ inline uint16_t f64_to_bf16(double d) {
 // constants), degree-13 Taylor polynomial of e^t on |t| <= ln2/2 by Horner
 // with explicit fma, scaling by 2^n. Uses IEEE basic operations only, so the
 // CPU restatement that follows the same steps produces the same bits.
-__device__ inline double exp_det(double r) {
-  if (r != r) return r;
-  if (r > 709.0) return __builtin_huge_val();
-  if (r < -690.0) return 0.0;
-  const double log2e = 1.4426950408889634074;
+// exp_steps: the steps after n = rint(r / ln2).
+__device__ inline double exp_steps(double r, double n) {
   const double ln2_hi = 6.93147180369123816490e-01;
   const double ln2_lo = 1.90821492927058770002e-10;
-  const double n = rint(r * log2e);
   double t = __builtin_fma(-n, ln2_hi, r);
   t = __builtin_fma(-n, ln2_lo, t);
   double p = 1.0 / 6227020800.0;
@@ -75,6 +71,14 @@ __device__ inline double exp_det(double r) {
   p = __builtin_fma(p, t, 1.0);
   p = __builtin_fma(p, t, 1.0);
   return ldexp(p, static_cast<int>(n));
+}
+
+constexpr double kExpLog2e = 1.4426950408889634074;
+__device__ inline double exp_det(double r) {
+  if (r != r) return r;
+  if (r > 709.0) return __builtin_huge_val();
+  if (r < -690.0) return 0.0;
+  return exp_steps(r, rint(r * kExpLog2e));
 }
 
 // bf16(sigmoid(v)) for a bf16-valued v, computed in fp64 and rounded once.

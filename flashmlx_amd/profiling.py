@@ -36,7 +36,7 @@ STAGE_OF = [
     (r"combine_kernel", "combine"),
     # the decoder stack's kernels (fmx_model)
     (r"attn_split_kernel", "attention (single token)"),
-    (r"attn_mfma_kernel|attn_kernel", "attention (several tokens)"),
+    (r"attn_tile_kernel|attn_kernel", "attention (several tokens)"),
     (r"dense_dec_kernel<true", "q/k/v with input norm"),
     (r"dense_dec_kernel<false", "q/k/v, o_proj"),
     (r"dense_wide_kernel", "lm_head"),

@@ -1,7 +1,8 @@
 """Attention of forwards with several tokens per sequence (causal, over the
-KV cache, model.cpp:874-884) against fp64, at the edges of its row tiles (16
-and 64 rows) and key blocks (64, 128, folds every 256 keys), for MHA and
-GQA, head sizes on the matrix-core kernel (64, 128) and off it (32).
+KV cache, model.cpp:874-884) against fp64, at row and key counts around
+multiples of 16 and 64, for MHA and GQA, head sizes on the matrix cores (64,
+128) and off them (32): what the result is worth. That it has the oracle's
+bits: test_gpu_attention_bits.py.
 
 The decoder layer is built so that its residual stream is the attention's
 output: no q projection (q is its bias, rotated), an identity o projection,
