@@ -538,13 +538,18 @@ hipError_t launch_attn_prefill(const AttnArgs& a, int T, hipStream_t stream) {
     // before the call: 32 tokens x 16 heads of 128 7 / 14, 19 / 26, 48 / 59,
     // 119 / 143; 48 x 16 8 / 15, 22 / 26, 62 / 60, 161 / 146; 64 x 16 13 / 15,
     // 31 / 26, 82 / 60, 206 / 146; heads of 64, 8 x 16 6 / 10, 13 / 16, 32 /
-    // 36, 78 / 85; 24 x 16 7 / 10, 16 / 16, 43 / 36, 108 / 87). A little
-    // beyond it rows are still faster over few keys.
+    // 36, 78 / 85; 24 x 16 7 / 10, 16 / 16, 43 / 36, 108 / 87). Over few keys
+    // rows are faster up to two rounds of them, one round for head size 64
+    // (96 x 16 of 128 at 0 / 32 / 64 keys before the call 16 / 17, 18 / 18,
+    // 22 / 20; 48 x 16 of 64 at 0 / 64 / 128 8 / 11, 10 / 13, 13 / 15; 64 x 16
+    // 12 / 12, 14 / 13, 19 / 14).
+    const bool hd128 = a.hd == 128;
     const int64_t n = static_cast<int64_t>(T) * a.nh;
     const int64_t resident = 256 * std::min<int64_t>(3, kLdsBytes / attn_row_lds(a.max_seq));
     const int64_t keys = a.offs ? a.max_seq : a.off + a.L;
-    const bool rows = n <= (a.hd == 128 ? resident : resident / 3) || (a.hd == 128 && n <= 1024 && keys <= 128);
-    if (!rows) return a.hd == 128 ? launch_tiles<128>(a, B, stream) : launch_tiles<64>(a, B, stream);
+    const int64_t most = keys <= (hd128 ? 128 : 192) ? (hd128 ? 2 * resident : resident)
+                                                     : (hd128 ? resident : resident / 3);
+    if (n > most) return hd128 ? launch_tiles<128>(a, B, stream) : launch_tiles<64>(a, B, stream);
   }
   const dim3 grid(T, a.nh);
   const size_t lds = attn_row_lds(a.max_seq);
