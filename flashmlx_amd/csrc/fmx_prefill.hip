@@ -71,6 +71,7 @@ constexpr int kPfMT = kPassRows / 16;                        // 16-row tiles per
 constexpr int kPfABytes = kPassRows * 256;                   // a pass's rows, one unit
 constexpr int kPfStages = 2;
 constexpr int kXcds = 8;  // MI355X: 8 XCDs, each with its own L2
+constexpr int kNarrowRows = 32;  // rows per pass of a narrow set, at most
 constexpr int64_t kL2Bytes = 4 << 20;
 constexpr int64_t kPassMajorBytes = 3 << 20;  // weights that stay beside the rows passing through
 
@@ -533,7 +534,8 @@ __device__ __attribute__((always_inline)) void pf_grid(const PfArgs& a, uint8_t*
   }
   if (rows <= 0) return;
   // one call site per tile count and arithmetic: each inlined copy is
-  // compiled on its own
+  // compiled on its own (narrow sets: passes of at most kNarrowRows rows,
+  // which launch_pf checks)
   static_assert(kPfMT == 4, "row-tile dispatch below covers passes of up to 4 tiles");
   bool exact;
   if (MLX && a.n_flag > 1) {
@@ -552,15 +554,23 @@ __device__ __attribute__((always_inline)) void pf_grid(const PfArgs& a, uint8_t*
     switch ((rows + 15) / 16) {
       case 1: pf_item<DUAL, 1, false, MLX, NARROW>(P, ng, row0, rows, e, ks, s_pf, a.f16_flag, a.flag_out); break;
       case 2: pf_item<DUAL, 2, false, MLX, NARROW>(P, ng, row0, rows, e, ks, s_pf, a.f16_flag, a.flag_out); break;
-      case 3: pf_item<DUAL, 3, false, MLX, NARROW>(P, ng, row0, rows, e, ks, s_pf, a.f16_flag, a.flag_out); break;
-      default: pf_item<DUAL, 4, false, MLX, NARROW>(P, ng, row0, rows, e, ks, s_pf, a.f16_flag, a.flag_out); break;
+      case 3:
+        if constexpr (!NARROW) pf_item<DUAL, 3, false, MLX, NARROW>(P, ng, row0, rows, e, ks, s_pf, a.f16_flag, a.flag_out);
+        break;
+      default:
+        if constexpr (!NARROW) pf_item<DUAL, 4, false, MLX, NARROW>(P, ng, row0, rows, e, ks, s_pf, a.f16_flag, a.flag_out);
+        break;
     }
   } else {
     switch ((rows + 15) / 16) {
       case 1: pf_item<DUAL, 1, true, MLX, NARROW>(P, ng, row0, rows, e, ks, s_pf, a.f16_flag, a.flag_out); break;
       case 2: pf_item<DUAL, 2, true, MLX, NARROW>(P, ng, row0, rows, e, ks, s_pf, a.f16_flag, a.flag_out); break;
-      case 3: pf_item<DUAL, 3, true, MLX, NARROW>(P, ng, row0, rows, e, ks, s_pf, a.f16_flag, a.flag_out); break;
-      default: pf_item<DUAL, 4, true, MLX, NARROW>(P, ng, row0, rows, e, ks, s_pf, a.f16_flag, a.flag_out); break;
+      case 3:
+        if constexpr (!NARROW) pf_item<DUAL, 3, true, MLX, NARROW>(P, ng, row0, rows, e, ks, s_pf, a.f16_flag, a.flag_out);
+        break;
+      default:
+        if constexpr (!NARROW) pf_item<DUAL, 4, true, MLX, NARROW>(P, ng, row0, rows, e, ks, s_pf, a.f16_flag, a.flag_out);
+        break;
     }
   }
 }
@@ -624,6 +634,8 @@ hipError_t launch_pf(const PfArgs& a, bool dual, hipStream_t stream) {
   const bool narrow = a.n_items0 ? a.s0.narrow : a.s1.narrow;
   if ((a.n_items0 && !a.s0.narrow == narrow) || (a.n_items1 && !a.s1.narrow == narrow) || (narrow && !mlx))
     return hipErrorInvalidValue;
+  for (const PfSet* s : {&a.s0, &a.s1})
+    if (s->narrow && (s->pass_n || s->pass_rows < 1 || s->pass_rows > kNarrowRows)) return hipErrorInvalidValue;
   if (narrow)
     hipLaunchKernelGGL(pf_gemm_mlx_narrow, dim3(n), dim3(kPfThreads), (kPfStages * pf_stage_bytes<false, true>()), stream,
                        a);
