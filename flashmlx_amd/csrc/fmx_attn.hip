@@ -219,13 +219,14 @@ __global__ __launch_bounds__(kAttnThreads) void attn_kernel(AttnArgs a) {
 //
 // Bound by the matrix cores' fp64 and fp32 rates (58 and 155 TFLOP/s,
 // measured): one sequence of 3001 tokens, 16 heads of 128, 18.4 GFLOP of
-// each, 433 us, took 737 us (the row kernel 3300); the difference are the
-// exps (75 us), the operands' preparation (3 VALU instructions per score
-// step, which do not overlap with the fp32 products) and the loads. With
-// the first pass in fp32 870 us. 1024 tokens 119 us (495 as rows), 512 tokens
-// behind 1024 cached ones 138 us (552). Two tiles at a time, or the next
-// tile's score steps between the value products, gave nothing: with two waves
-// per SIMD the chains are covered.
+// each, 433 us, took 697-751 us (averages on several boxes; the row kernel
+// 3300-3440). Without the exps it was 75 us less, without the loads 75,
+// without the value products 260; the rest is the scores, whose operands'
+// preparation (2 VALU instructions per step, 3 with the exchange) is not
+// hidden behind the fp32 products. With the first pass in fp32 870-890 us.
+// 1024 tokens 119 us (495 as rows), 512 tokens behind 1024 cached ones 138
+// us (552). Two key tiles at a time, or the next tile's score steps between
+// the value products, gave nothing: two waves per SIMD cover the chains.
 constexpr int kTileRows = 16;
 
 // exp_det of r <= 0 or NaN without branches, so that several run side by
@@ -543,13 +544,18 @@ hipError_t launch_attn_prefill(const AttnArgs& a, int T, hipStream_t stream) {
     // (96 x 16 of 128 at 0 / 32 / 64 keys before the call 16 / 17, 18 / 18,
     // 22 / 20; 48 x 16 of 64 at 0 / 64 / 128 8 / 11, 10 / 13, 13 / 15; 64 x 16
     // 12 / 12, 14 / 13, 19 / 14).
+    // Rows are also faster where a tile has only two of them, over few keys
+    // three (96 sequences x 16 heads of 128 over 100 / 500 / 2000 keys, 2 rows
+    // 38 / 60, 139 / 154, 519 / 537; 3 rows 54 / 60, 189 / 151, 720 / 529;
+    // heads of 64, 2 rows 32 / 42, 97 / 91, 374 / 319).
     const bool hd128 = a.hd == 128;
     const int64_t n = static_cast<int64_t>(T) * a.nh;
+    const int64_t tiles = static_cast<int64_t>((a.L + kTileRows - 1) / kTileRows) * a.nh * B;
     const int64_t resident = 256 * std::min<int64_t>(3, kLdsBytes / attn_row_lds(a.max_seq));
-    const int64_t keys = a.offs ? a.max_seq : a.off + a.L;
-    const int64_t most = keys <= (hd128 ? 128 : 192) ? (hd128 ? 2 * resident : resident)
-                                                     : (hd128 ? resident : resident / 3);
-    if (n > most) return hd128 ? launch_tiles<128>(a, B, stream) : launch_tiles<64>(a, B, stream);
+    const bool few_keys = (a.offs ? a.max_seq : a.off + a.L) <= (hd128 ? 128 : 192);
+    const int64_t most = hd128 ? (few_keys ? 2 * resident : resident) : (few_keys ? resident : resident / 3);
+    const int per_tile = (hd128 ? 3 : 2) + (few_keys ? 1 : 0);  // rows that take a tile's time
+    if (n > most && n >= per_tile * tiles) return hd128 ? launch_tiles<128>(a, B, stream) : launch_tiles<64>(a, B, stream);
   }
   const dim3 grid(T, a.nh);
   const size_t lds = attn_row_lds(a.max_seq);

@@ -90,7 +90,7 @@ def _ids(g, B, L, hi=V):
 # few rows (rows x heads, by the caches' length): the row kernel; the others in tiles
 @pytest.mark.parametrize("nh,nkv,hd,B,L,ctx", [
     (4, 4, 128, 1, 2, 0), (16, 16, 128, 1, 17, 111), (4, 2, 32, 1, 40, 30), (4, 4, 64, 2, 9, 60),
-    (32, 8, 128, 25, 2, 0), (32, 8, 128, 17, 3, 61), (16, 2, 128, 3, 48, 16), (16, 16, 128, 1, 65, 64),
+    (32, 8, 128, 13, 4, 0), (32, 8, 128, 13, 4, 61), (32, 8, 128, 9, 3, 260), (16, 2, 128, 3, 48, 16), (16, 16, 128, 1, 65, 64),
     (32, 4, 128, 1, 33, 4060), (8, 2, 128, 1, 130, 301), (16, 4, 128, 1, 1030, 0),
     (8, 2, 64, 6, 7, 500), (32, 2, 64, 5, 5, 95), (8, 8, 64, 1, 300, 0), (16, 16, 64, 1, 1025, 700), (32, 8, 64, 2, 257, 63)])
 def test_attention_bits(gpu, fmx, oracle, nh, nkv, hd, B, L, ctx):
