@@ -234,9 +234,10 @@ __global__ __launch_bounds__(256) void dense_dec_kernel(DenseArgs a) {
 // holds its waves' activation operands in registers across them and issues a
 // tile's weights before it multiplies the tile before, so the weight stream
 // never waits for a workgroup's start, its rows or its reduction. Bound by
-// HBM: lm_head [151936, 2048] (175 MB) 44.0 -> 34.5 us for one row (5.1 TB/s,
-// a large copy's rate), 59-61 -> 38.0 us for 8 rows, which every tile's
-// workgroup read again. From two tiles per resident workgroup on: below, a
+// HBM: lm_head [151936, 2048] (175 MB) 44 -> 34-37 us for one row (averages of
+// two traces; 4.8-5.1 TB/s, where a large copy has 5.1 and streams that only
+// read 5.3-6.2), 59-61 -> 39-40 us for 8 rows, which every tile's workgroup
+// read again. From two tiles per resident workgroup on: below, a
 // workgroup has one tile or the grid one round, and nothing to overlap.
 constexpr int kDnWideWgs = 3 * 256;  // resident workgroups: 3 per CU by registers
 constexpr int kDnWideTiles = 2 * kDnWideWgs;
