@@ -73,6 +73,7 @@ constexpr int kPfStages = 2;
 constexpr int kXcds = 8;  // MI355X: 8 XCDs, each with its own L2
 constexpr int kNarrowRows = 32;  // rows per pass of a narrow set, at most
 constexpr int64_t kL2Bytes = 4 << 20;
+constexpr int kPassMajorItems = 512;          // work items of a grid, two per CU
 constexpr int64_t kPassMajorBytes = 3 << 20;  // weights that stay beside the rows passing through
 
 // Packed blocks per wave: one gate/up pair or two single blocks (2 KB of
@@ -484,7 +485,12 @@ __device__ __attribute__((always_inline)) void pf_item(const PfSet& P, int ng, i
 // again: at 4096 tokens, 16.8 MB per group, the gate/up grid missed the L2
 // 16.4 M times instead of 6.1 M and the block took 793 us instead of 768.)
 // Otherwise it runs every pass of one group back to back, so the group's
-// weights are fetched once (rows that fit, 512 tokens: 0.5-0.9 % faster so).
+// weights are fetched once (rows that fit, 512 tokens: 0.5-0.9 % faster so),
+// and so does a grid of at most two items per CU, all of which run at the
+// same time (quantized_matmul, one pass after the other -> one group after
+// the other: [2048, 5632] 700 rows, 352 items, 61.7 -> 54.8 us, 2000 rows, 512
+// items, 82 -> 79; [4096, 8192] 300 rows 74.3 -> 66.8; but [4096, 5632] 1100
+// rows, 576 items, 99.2 -> 102.4, [2048, 2048] 3001 rows, 752, 48.8 -> 51.0).
 // Blocks past the work (padding, passes the sort did not fill) exit.
 template <bool DUAL, bool MLX, bool NARROW>
 __device__ __attribute__((always_inline)) void pf_grid(const PfArgs& a, uint8_t* s_pf) {
@@ -636,15 +642,17 @@ hipError_t launch_pf(const PfArgs& a, bool dual, hipStream_t stream) {
     return hipErrorInvalidValue;
   for (const PfSet* s : {&a.s0, &a.s1})
     if (s->narrow && (s->pass_n || s->pass_rows < 1 || s->pass_rows > kNarrowRows)) return hipErrorInvalidValue;
+  PfArgs g = a;
+  if (n <= kPassMajorItems) g.s0.pass_major = g.s1.pass_major = 0;
   if (narrow)
     hipLaunchKernelGGL(pf_gemm_mlx_narrow, dim3(n), dim3(kPfThreads), (kPfStages * pf_stage_bytes<false, true>()), stream,
-                       a);
+                       g);
   else if (dual)
-    hipLaunchKernelGGL(pf_gemm<true>, dim3(n), dim3(kPfThreads), pf_lds_bytes(true), stream, a);
+    hipLaunchKernelGGL(pf_gemm<true>, dim3(n), dim3(kPfThreads), pf_lds_bytes(true), stream, g);
   else if (mlx)
-    hipLaunchKernelGGL(pf_gemm_mlx, dim3(n), dim3(kPfThreads), pf_lds_bytes(false), stream, a);
+    hipLaunchKernelGGL(pf_gemm_mlx, dim3(n), dim3(kPfThreads), pf_lds_bytes(false), stream, g);
   else
-    hipLaunchKernelGGL(pf_gemm<false>, dim3(n), dim3(kPfThreads), pf_lds_bytes(false), stream, a);
+    hipLaunchKernelGGL(pf_gemm<false>, dim3(n), dim3(kPfThreads), pf_lds_bytes(false), stream, g);
   return hipGetLastError();
 }
 

@@ -46,3 +46,22 @@ def test_nh_block_rows_beyond_l2(gpu, fmx, oracle):
         np.testing.assert_array_equal(y[lo:hi], from_dev_bf16(block(xd[lo:hi].contiguous())), err_msg=f"rows {lo}..")
     ref, _, _ = oracle.nh_moe_block(cfg.oracle_cfg(), N.host_weights(w), np.ascontiguousarray(x[ROWS]), oracle.ACC_F64)
     print(assert_close_rows(y[ROWS], ref, "rows beyond an L2"))
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
+def test_quantized_matmul_rows_beyond_l2(gpu, fmx, dtype):
+    """One set alone, on both sides of the 512 work items from which it runs
+    one pass after the other (45 column groups)."""
+    import torch
+    from flashmlx_amd import moe as Mo
+    N, K = 5648, 2048
+    dt = getattr(torch, dtype)
+    g = torch.Generator(device="cuda").manual_seed(45)
+    w = torch.randint(-2**31, 2**31, (N, K // 8), generator=g, device="cuda", dtype=torch.int64).to(torch.int32)
+    s = (torch.rand((N, K // 64), generator=g, device="cuda") * 0.01 + 0.002).to(dt)
+    b = (torch.randn((N, K // 64), generator=g, device="cuda") * 0.05).to(dt)
+    x = torch.randn((1105, K), generator=g, device="cuda").to(dt)
+    y = Mo.quantized_matmul(x, w, s, b)
+    for lo, hi in [(0, 600), (505, 1105), (1024, 1105)]:
+        part = Mo.quantized_matmul(x[lo:hi].contiguous(), w, s, b)
+        assert torch.equal(y[lo:hi].view(torch.int16), part.view(torch.int16)), f"rows {lo}.."
