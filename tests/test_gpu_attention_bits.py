@@ -99,7 +99,7 @@ def test_attention_bits(gpu, fmx, oracle, nh, nkv, hd, B, L, ctx):
     _run(oracle, cfg, w, dm, _ids(g, B, L), ctx, [ctx] * B)
 
 
-@pytest.mark.parametrize("nh,L", [(4, 37), (32, 19)])
+@pytest.mark.parametrize("nh,L", [(4, 37), (32, 37)])
 def test_attention_bits_sequence_offsets(gpu, fmx, oracle, nh, L):
     """Several tokens per sequence at per-sequence device offsets."""
     import torch
