@@ -237,10 +237,13 @@ __global__ __launch_bounds__(256) void dense_dec_kernel(DenseArgs a) {
 // HBM: lm_head [151936, 2048] (175 MB) 44 -> 34-37 us for one row (averages of
 // two traces; 4.8-5.1 TB/s, where a large copy has 5.1 and streams that only
 // read 5.3-6.2), 59-61 -> 39-40 us for 8 rows, which every tile's workgroup
-// read again. From two tiles per resident workgroup on: below, a
-// workgroup has one tile or the grid one round, and nothing to overlap.
+// read again. From two tiles per resident workgroup on (below, a
+// workgroup has one tile or the grid one round, and nothing to overlap), for
+// up to four rows, which the other kernel reads again cheaply, from three
+// (one-layer step, before -> this kernel: [25600, 512] 1 row 41.2 -> 42.5 us,
+// 16 rows 62.7 -> 61.5; [25600, 2048] 47.5 -> 48.4, 71.7 -> 68.8; [49152,
+// 2048] 53.6 -> 51.4, 82.2 -> 72.8).
 constexpr int kDnWideWgs = 3 * 256;  // resident workgroups: 3 per CU by registers
-constexpr int kDnWideTiles = 2 * kDnWideWgs;
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void dense_wide_kernel(DenseArgs a) {
   __shared__ f32x4_t s_acc[2][3][kWave];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -910,7 +913,7 @@ hipError_t launch_dense_dec(const DenseArgs& a, hipStream_t stream) {
   const size_t lds = nin ? static_cast<size_t>(a.T) * a.nu * 128 * 2 : 0;
   if (nin)
     hipLaunchKernelGGL(dense_dec_kernel<true>, dim3(a.nt), dim3(256), lds, stream, a);
-  else if (a.nt >= kDnWideTiles && a.nu <= 4 * kDnBatch && !a.bias && !a.res)
+  else if (a.nt >= (a.T > 4 ? 2 : 3) * kDnWideWgs && a.nu <= 4 * kDnBatch && !a.bias && !a.res)
     // as many workgroups as make every one's tile count the same
     hipLaunchKernelGGL(dense_wide_kernel, dim3((a.nt + (a.nt + kDnWideWgs - 1) / kDnWideWgs - 1) /
                                                ((a.nt + kDnWideWgs - 1) / kDnWideWgs)),

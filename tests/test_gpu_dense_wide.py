@@ -1,5 +1,5 @@
-"""The lm_head of decode batches on the kernel for many tiles (1536 and more,
-each workgroup several tiles) against the one-tile-per-workgroup kernel: every
+"""The lm_head of decode batches on the kernel for many tiles (1536 and more, for
+up to 4 rows 2304; each workgroup several tiles) against the one-tile-per-workgroup kernel: every
 logit is the same sum in the same order, so the logits of a vocabulary slice
 have the bits of a model whose lm_head is that slice alone."""
 from __future__ import annotations
@@ -15,8 +15,9 @@ from test_gpu_model import _tiny_cfg
 pytestmark = pytest.mark.gpu
 
 
-# fewest tiles of the kernel, an uneven last round, one tile more; K of 1, 9
-# and 16 units (waves without a unit, with unequal ones, with four)
+# fewest tiles of the kernel (16 rows; up to 4 rows from 2304 tiles on), an
+# uneven last round, one tile more; K of 4, 9 and 16 units (waves with one
+# unit, with unequal ones, with four)
 @pytest.mark.parametrize("V,H", [(1536 * 16, 512), (2305 * 16, 1152), (1537 * 16, 2048)])
 def test_wide_lm_head_equals_slices(gpu, fmx, V, H):
     import torch
