@@ -3,7 +3,7 @@ from __future__ import annotations
 
 import numpy as np
 
-# Parity bar for bf16 outputs (north-star tolerance), plus a tight relative
+# Parity bar for bf16 outputs, plus a tight relative
 # bound that makes small-magnitude outputs meaningful.
 RTOL = 2e-2
 ATOL = 1e-2
